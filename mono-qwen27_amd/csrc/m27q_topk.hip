@@ -395,68 +395,73 @@ __global__ __launch_bounds__(kTopkSelBlock) void k_topk_select(const float *__re
     }
 }
 
+// Sum of p over lanes 0 .. k - 1 in lane order, rounded as a sequential loop
+// from 0 rounds; `prefix` gets, in lane i, the sum through lane i.  Each lane's
+// value comes through a scalar register (v_readlane), so a step of the chain is
+// one add.  Steps past k add the 0 those lanes hold, which changes nothing.
+__device__ __forceinline__ float ordered_sum(float p, int k, int lane, float &prefix) {
+    constexpr int B = 16;
+    float s = 0.f;
+    prefix = 0.f;
+    for (int i0 = 0; i0 < k; i0 += B) {
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), i0 + i));
+            prefix = lane == i0 + i ? s : prefix;
+        }
+    }
+    return s;
+}
+
 // Sampling from the top-k candidates, in the steps and order of sample()
 // (src/mono27b_chat.cpp:203-270) after its top-k: probabilities
-// e^((v_i - v_0) / T) computed per lane (exp_cw; 0 below e^-87, NaN kept),
-// then one lane runs the sum, the normalization, the min_p and top_p cuts and
-// the pick in candidate order, so the float sums round as the reference's
-// sequential loop does.
+// e^((v_i - v_0) / T) (exp_cw; 0 below e^-87, NaN kept), the sum, the
+// normalization, the min_p and top_p cuts and the pick.  One wave, candidate i
+// in lane i.  The float sums run in candidate order (ordered_sum), so they
+// round as the reference's sequential loop does; the cuts and the pick only
+// compare each candidate's own running sum, so one prefix sum over the kept
+// candidates serves top_p's cut, the total (its value at the last candidate
+// kept) and the pick.  Bound by the latency of its 2 k dependent adds: 64
+// candidates took 21.7 us with one lane walking LDS (five loops of dependent
+// reads and 64 divides), 5.6 us so (kernel trace).
 __global__ __launch_bounds__(kWave) void k_sample(const int32_t *__restrict__ idx, const float *__restrict__ val,
                                                   int k, float temperature, float min_p, float top_p,
                                                   const float *__restrict__ u, int32_t *__restrict__ token) {
-    __shared__ float p[kTopkMaxK];
-    __shared__ int kept[kTopkMaxK];
+    static_assert(kTopkMaxK == kWave, "one candidate per lane");
     const int lane = (int)threadIdx.x;
-    const int best = idx[0];
-    if (!(temperature > 0.f)) {
-        if (lane == 0) *token = best;
-        return;
-    }
-    if (lane < k) {
-        const float a = (val[lane] - val[0]) / temperature;
-        p[lane] = a >= -87.0f ? exp_cw(a) : (a < -87.0f ? 0.0f : a);
-    }
-    __syncthreads();
-    if (lane != 0) return;
-    float sum = 0.f;
-    for (int i = 0; i < k; ++i) sum += p[i];
-    if (!(sum > 0.f) || !isfinite(sum)) {
-        *token = best;
-        return;
-    }
-    for (int i = 0; i < k; ++i) p[i] /= sum;
-    // min_p: drop candidates below p_0 * min_p (kept in order); p_0 itself
-    // always stays unless min_p > 1, and then the pick falls back to best.
-    const float thresh = p[0] * min_p;
-    int n = 0;
-    for (int i = 0; i < k; ++i)
-        if (!(p[i] < thresh)) kept[n++] = i;
-    if (n == 0) {
-        *token = best;
-        return;
-    }
-    if (top_p < 1.f) {
-        float acc = 0.f;
-        for (int i = 0; i < n; ++i) {
-            acc += p[kept[i]];
-            if (acc >= top_p) {
-                n = i + 1;
-                break;
+    const bool in = lane < k;
+    const int src = in ? lane : 0;
+    const int id = idx[src];
+    const float v = val[src], v0 = val[0], rnd = *u;
+    const int best = __builtin_amdgcn_readfirstlane(id);
+    int pick_id = best;
+    if (temperature > 0.f) {
+        const float a = (v - v0) / temperature;
+        float p = a >= -87.0f ? exp_cw(a) : (a < -87.0f ? 0.0f : a);
+        p = in ? p : 0.f;
+        float prefix;
+        const float sum = ordered_sum(p, k, lane, prefix);
+        if (sum > 0.f && isfinite(sum)) {
+            p /= sum;
+            // min_p: drop candidates below p_0 * min_p; p_0 itself always
+            // stays unless min_p > 1, and then the pick falls back to best.
+            const float thresh = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(p))) * min_p;
+            bool kept = in && !(p < thresh);
+            uint64_t m = __ballot(kept);
+            if (m) {
+                ordered_sum(kept ? p : 0.f, k, lane, prefix);
+                if (top_p < 1.f) {  // cut after the first candidate whose running sum reaches top_p
+                    const uint64_t reach = __ballot(kept && prefix >= top_p);
+                    if (reach) m &= (reach & (0ull - reach)) * 2 - 1;
+                }
+                const int last = 63 - __clzll((long long)m);
+                const float pick = rnd * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(prefix), last));
+                const uint64_t hit = __ballot(kept && pick <= prefix) & m;
+                pick_id = __builtin_amdgcn_readlane(id, hit ? __ffsll((long long)hit) - 1 : last);
             }
         }
     }
-    float total = 0.f;
-    for (int i = 0; i < n; ++i) total += p[kept[i]];
-    const float pick = *u * total;
-    float run = 0.f;
-    for (int i = 0; i < n; ++i) {
-        run += p[kept[i]];
-        if (pick <= run) {
-            *token = idx[kept[i]];
-            return;
-        }
-    }
-    *token = idx[kept[n - 1]];
+    if (lane == 0) *token = pick_id;
 }
 
 hipError_t launch_sample(const int32_t *idx, const float *val, int k, float temperature, float min_p, float top_p,

@@ -131,3 +131,24 @@ def test_sample_matches_oracle(m27q, ora, dev, T, min_p, top_p):
         want = ora.sample(idx, val, T, min_p, top_p, float(u))
         m27q.sample(di, dv, k, T, min_p, top_p, to_dev(np.array([u], np.float32), dev), tok)
         assert int(to_host(tok)[0]) == want, float(u)
+
+
+@pytest.mark.parametrize("k,T,min_p,top_p", [(1, 0.8, 0.05, 0.95), (15, 2.0, 0.0, 0.9), (17, 1.5, 0.2, 1.0),
+                                             (64, 3.0, 0.0, 0.999), (64, 3.0, 1.5, 0.95), (33, 1.0, 0.0, 1e-6)])
+def test_sample_candidate_counts(m27q, ora, dev, k, T, min_p, top_p):
+    """One candidate per lane: candidate counts around the 16-step chunks of the
+    running sums (1, 15, 17, 33, 64), a min_p above 1 (nothing kept: the first
+    candidate) and a top_p that the first candidate reaches alone; unused
+    candidates behind the first k hold values that would win."""
+    import torch
+    rng = np.random.default_rng(k)
+    val = np.sort(rng.standard_normal(64).astype(np.float32))[::-1].copy()
+    val[k:] = 50.0
+    idx = rng.permutation(1000)[:64].astype(np.int32)
+    di, dv = to_dev(idx, dev), to_dev(val, dev)
+    tok = torch.empty(1, dtype=torch.int32, device=dev)
+    say("sample counts", k, T, min_p, top_p)
+    for u in list(np.linspace(0.0, 0.9999, 80, dtype=np.float32)) + [np.float32(1.0)]:
+        want = ora.sample(idx[:k], val[:k], T, min_p, top_p, float(u))
+        m27q.sample(di, dv, k, T, min_p, top_p, to_dev(np.array([u], np.float32), dev), tok)
+        assert int(to_host(tok)[0]) == want, float(u)
