@@ -213,7 +213,8 @@ m27q_status gemv_impl(int n, const m27q_weight *ws, const void *xq, const float 
 // GGUF-layout weights take the same few-token kernel (with temporal loads);
 // from M = 3, GGUF-layout Q4_K / Q5_K / Q6_K take the MFMA kernel (staged from
 // the row blocks), GGUF-layout Q8_0 and IQ4_XS one launch per matrix of the
-// VALU kernel (m27q_matmul.hip).
+// VALU kernel (m27q_matmul.hip).  More rows take the wide kernel (m27q_wide.h,
+// matmul_wide_wins).
 constexpr int kMtMaxM = 2;
 constexpr size_t kMtLdsBudget = 80 * 1024;  // two workgroups per CU
 
@@ -239,7 +240,10 @@ m27q_status matmul_multi_impl(int n, const m27q_weight *ws, int M, const void *x
     const ActView a = act_view(xq, M, p.K);
     const bool few = M <= kMtMaxM && (M == 1 || !matmul_mfma_direct(type, layout)) &&
                      matmul_mt_lds_bytes(type, p.upr) <= kMtLdsBudget;
-    if (!few && !matmul_mfma_takes(type, layout)) {  // GGUF Q8_0 / IQ4_XS from M = 3
+    long long sets = 0;
+    for (int i = 0; i < n; ++i) sets += ((long long)ws[i].row_count + 15) / 16;
+    const bool wide = !few && lds_limit() >= kWideLds && matmul_wide_wins(type, layout, sets, M, cu_count());
+    if (!few && !wide && !matmul_mfma_takes(type, layout)) {  // GGUF Q8_0 / IQ4_XS of a few rows
         if (dry) return M27Q_OK;
         for (int i = 0; i < n; ++i) {
             MatmulParams q{};
@@ -254,7 +258,7 @@ m27q_status matmul_multi_impl(int n, const m27q_weight *ws, int M, const void *x
             q.xs = a.s;
             q.Y = Ys[i];
             q.res = res[i];
-            const hipError_t e = launch_matmul_q8(type, layout, q, stream);
+            const hipError_t e = launch_matmul_q8(type, q, stream);
             if (e != hipSuccess) return hip_status(e);
         }
         return M27Q_OK;
@@ -262,8 +266,9 @@ m27q_status matmul_multi_impl(int n, const m27q_weight *ws, int M, const void *x
     if (!few && matmul_mfma_lds_bytes(type) > lds_limit()) return M27Q_ERR_SHAPE;
     // The MFMA kernel reads each matrix through a buffer descriptor with a
     // 32-bit size; the activations (M <= kMaxM rows of K <= kMaxK) stay far
-    // below it.
-    for (int i = 0; i < n && !few; ++i) {
+    // below it.  (The wide kernel's descriptors cover 16 rows each; GGUF Q8_0
+    // and IQ4_XS, which the MFMA kernel does not take, have no such limit.)
+    for (int i = 0; i < n && !few && matmul_mfma_takes(type, layout); ++i) {
         const size_t wb = tiled ? tiled_bytes(type, ws[i].row_blocks, ws[i].row_count)
                                 : (size_t)ws[i].row_blocks * ws[i].row_count * (size_t)block_bytes(type);
         if (wb >= (1ull << 32)) return M27Q_ERR_SHAPE;
@@ -280,7 +285,9 @@ m27q_status matmul_multi_impl(int n, const m27q_weight *ws, int M, const void *x
         p.res[i] = res[i];
         p.rc[i] = (int)ws[i].row_count;
     }
-    return hip_status(few ? launch_matmul_mt(type, layout, p, stream) : launch_matmul_mfma(type, layout, p, stream));
+    return hip_status(few    ? launch_matmul_mt(type, layout, p, stream)
+                      : wide ? launch_matmul_wide(type, layout, p, stream)
+                             : launch_matmul_mfma(type, layout, p, stream));
 }
 
 // Up to kMaxMulti weights of one K sharing one activation, of any mix of

@@ -1,7 +1,8 @@
-// m27q_matmul.hip -- small-M products Y[M][N] = X[M][K] W[N][K]^T, M <= 64.
+// m27q_matmul.hip -- products of up to 8 rows on GGUF-layout Q8_0 / IQ4_XS weights
+// (matmul_wide_wins): Y[M][N] = X[M][K] W[N][K]^T.
 //
 // Same wavefront tiling as the M = 1 GEMV (8 rows per wave, 16-byte weight
-// loads); the weights are read once per group of up to 16 activation rows and
+// loads); the weights are read once per group of up to 8 activation rows and
 // each lane keeps one accumulator per row.  Activations are staged in LDS per
 // K-chunk of 4 units for all rows of the group, so LDS stays small at any K.
 // No reference counterpart: the reference feeds prefill one token at a time
@@ -95,32 +96,23 @@ static hipError_t launch_mt(const MatmulParams &p, int m0, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <class T, int LAYOUT>
+template <class T>
 static hipError_t launch_m(const MatmulParams &p, hipStream_t s) {
-    for (int m0 = 0; m0 < p.M; m0 += 16) {
+    constexpr int L = M27Q_LAYOUT_GGUF;
+    for (int m0 = 0; m0 < p.M; m0 += 8) {
         const int left = p.M - m0;
-        hipError_t e;
-        if (left <= 2) e = launch_mt<T, LAYOUT, 2>(p, m0, s);
-        else if (left <= 4) e = launch_mt<T, LAYOUT, 4>(p, m0, s);
-        else if (left <= 8) e = launch_mt<T, LAYOUT, 8>(p, m0, s);
-        else e = launch_mt<T, LAYOUT, 16>(p, m0, s);
+        const hipError_t e = left <= 2   ? launch_mt<T, L, 2>(p, m0, s)
+                             : left <= 4 ? launch_mt<T, L, 4>(p, m0, s)
+                                         : launch_mt<T, L, 8>(p, m0, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
 
-template <class T>
-static hipError_t launch_l(const MatmulParams &p, int layout, hipStream_t s) {
-    return layout == M27Q_LAYOUT_TILED ? launch_m<T, M27Q_LAYOUT_TILED>(p, s) : launch_m<T, M27Q_LAYOUT_GGUF>(p, s);
-}
-
-hipError_t launch_matmul_q8(uint32_t type, int layout, const MatmulParams &p, hipStream_t s) {
+hipError_t launch_matmul_q8(uint32_t type, const MatmulParams &p, hipStream_t s) {
     switch (type) {
-        case kQ4_K: return launch_l<Q4K>(p, layout, s);
-        case kQ5_K: return launch_l<Q5K>(p, layout, s);
-        case kQ6_K: return launch_l<Q6K>(p, layout, s);
-        case kQ8_0: return launch_l<Q80>(p, layout, s);
-        case kIQ4_XS: return launch_l<IQ4XS>(p, layout, s);
+        case kQ8_0: return launch_m<Q80>(p, s);
+        case kIQ4_XS: return launch_m<IQ4XS>(p, s);
         default: return hipErrorInvalidValue;
     }
 }

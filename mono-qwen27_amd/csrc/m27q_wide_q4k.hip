@@ -1,0 +1,9 @@
+// m27q_wide_q4k.hip -- the instances of m27q_wide.h for one weight type (one
+// file per type, so that they compile in parallel).
+#include "m27q_wide.h"
+
+namespace m27q {
+
+hipError_t launch_wide_q4k(int layout, const MatmulMultiParams &p, hipStream_t s) { return launch_wide_l<WQ4K<false>>(layout, p, s); }
+
+}  // namespace m27q

@@ -206,3 +206,97 @@ def test_gguf_two_byte_aligned_base(m27q, ora, dev, type_name, rc, k):
             qf, df, sf = ora.quant_act(X[0])
             want, nrm = ora.gemv_act(t, wb, rb, rc, qf, df, sf)
             assert (np.abs(to_host(y).astype(np.float64) - want) <= int_dot_tol(nrm)).all(), "fp32 x"
+
+
+WIDE = [  # type, rows, K, M, layout: the wide kernel's launch shapes on 256 CUs (16-row sets per CU)
+    # up to one set per CU (K over 8 waves): one partial set, K of one unit
+    # (seven waves without work), a unit count the slices do not divide
+    ("Q4_K", 13, 256, 17, 1), ("Q5_K", 40, 2304, 33, 0), ("Q6_K", 40, 2304, 64, 1), ("Q6_K", 13, 256, 49, 0),
+    ("IQ4_XS", 40, 512, 64, 1), ("Q8_0", 13, 32, 17, 1), ("Q8_0", 40, 1056, 64, 1), ("Q8_0", 13, 160, 9, 0),
+    ("Q8_0", 13, 32, 5, 0), ("IQ4_XS", 13, 256, 5, 0),
+    # two row waves of at most one set: an odd set count (257: a wave without a
+    # set), a partial last 8-row tile and set
+    ("Q4_K", 4100, 1024, 33, 1), ("Q4_K", 4100, 256, 64, 0), ("Q5_K", 4100, 512, 48, 1), ("Q6_K", 4100, 768, 64, 0),
+    ("Q6_K", 8185, 512, 64, 1), ("IQ4_XS", 4100, 512, 37, 0), ("Q8_0", 4100, 160, 64, 0), ("Q8_0", 4100, 288, 33, 1),
+    # two row waves of up to three sets (2.0 to 6 sets per CU)
+    ("Q4_K", 8210, 512, 64, 1), ("Q5_K", 12301, 256, 17, 0), ("Q6_K", 24570, 256, 64, 1), ("Q8_0", 12301, 96, 47, 0),
+    ("IQ4_XS", 8210, 512, 64, 0),
+    # four row waves of up to three sets: just above 6 sets per CU, two rounds
+    ("Q4_K", 24600, 512, 64, 1), ("Q5_K", 50001, 256, 33, 1), ("Q6_K", 24600, 256, 33, 0), ("Q8_0", 24600, 160, 64, 1),
+    ("IQ4_XS", 24600, 256, 20, 0), ("Q4_K", 24600, 256, 17, 0),
+]
+
+
+@pytest.mark.parametrize("type_name,rc,k,M,layout", WIDE)
+def test_wide_vs_oracle(m27q, ora, dev, type_name, rc, k, M, layout):
+    """One launch of up to 64 rows (its first, last and tile-edge tokens, with a
+    residual) against the integer-dot oracle.  The scaled integer sums are
+    exact, so what differs is the order of the fp32 sums over groups and
+    blocks: the bar of every product (int_dot_tol)."""
+    import torch
+    t = getattr(m27q, type_name)
+    rb = k // m27q.BLOCK_ELEMS[t]
+    wb = ora.synth_weights(t, rc, k, seed=41)
+    w = m27q.Weight.upload(wb.reshape(-1), t, rb, rc, layout, dev)
+    X = np.random.default_rng(M).standard_normal((M, k)).astype(np.float32)
+    X[:, : k // 2] *= 1000.0  # groups of very different scale
+    act = m27q.Act(M, k, dev)
+    m27q.quant_act(to_dev(X, dev), act)
+    res = np.random.default_rng(M + 1).standard_normal((M, rc)).astype(np.float32)
+    Y = torch.full((M + 1, rc), 7.0, dtype=torch.float32, device=dev)
+    say("wide", type_name, rc, k, M, layout)
+    m27q.matmul_q8(w, act, Y[:M], residual=to_dev(res, dev))
+    got = to_host(Y).astype(np.float64)
+    assert (got[M] == 7.0).all()  # nothing written past the rows
+    q, d, s = act_host(m27q, act)
+    for m in sorted({0, min(15, M - 1), max(0, M // 16 * 16 - 1), min(M - 1, M // 16 * 16), M - 1}):
+        want, nrm = ora.gemv_act(t, wb, rb, rc, q[m], d[m], s[m])
+        assert (np.abs(got[m] - res[m] - want) <= int_dot_tol(nrm) + 1e-6 * np.abs(res[m])).all(), m
+
+
+@pytest.mark.parametrize("shapes,M", [((6144, 1024, 1024), 64), ((100, 17, 3000, 2000), 33), ((9000, 9000, 9000), 48)])
+def test_wide_multi_vs_oracle(m27q, ora, dev, shapes, M):
+    """Several weights in one wide launch: workgroups whose sets belong to
+    different weights, partial last sets in the middle of the run."""
+    import torch
+    k = 768
+    for name in ("Q4_K", "Q6_K"):
+        t = getattr(m27q, name)
+        wbs = [ora.synth_weights(t, rc, k, seed=70 + i) for i, rc in enumerate(shapes)]
+        ws = [m27q.Weight.upload(wb.reshape(-1), t, 3, rc, m27q.TILED, dev) for wb, rc in zip(wbs, shapes)]
+        X = np.random.default_rng(M + 7).standard_normal((M, k)).astype(np.float32)
+        act = m27q.Act(M, k, dev)
+        m27q.quant_act(to_dev(X, dev), act)
+        Ys = [torch.empty((M, rc), dtype=torch.float32, device=dev) for rc in shapes]
+        say("wide multi", name, shapes, M)
+        m27q.matmul_q8_multi(ws, act, Ys)
+        q, d, s = act_host(m27q, act)
+        for wb, rc, Y in zip(wbs, shapes, Ys):
+            got = to_host(Y).astype(np.float64)
+            for m in (0, M // 2, M - 1):
+                want, nrm = ora.gemv_act(t, wb, 3, rc, q[m], d[m], s[m])
+                assert (np.abs(got[m] - want) <= int_dot_tol(nrm)).all(), (name, rc, m)
+
+
+@pytest.mark.parametrize("type_name,rc,k", [("Q6_K", 1030, 2304), ("Q6_K", 8210, 768), ("Q8_0", 515, 1056)])
+def test_wide_two_byte_aligned_base(m27q, ora, dev, type_name, rc, k):
+    """GGUF Q6_K / Q8_0 weights 2 bytes past a multiple of 4 on the wide kernel."""
+    import torch
+    t = getattr(m27q, type_name)
+    rb = k // m27q.BLOCK_ELEMS[t]
+    wb = ora.synth_weights(t, rc, k, seed=92)
+    raw = torch.from_numpy(wb.reshape(-1).copy()).to(dev)
+    buf = torch.zeros(raw.numel() + 2, dtype=torch.uint8, device=dev)
+    buf[2:] = raw
+    w = m27q.Weight(buf[2:], t, rb, rc, m27q.GGUF)
+    M = 40
+    act = m27q.Act(M, k, dev)
+    m27q.quant_act(to_dev(np.random.default_rng(3).standard_normal((M, k)).astype(np.float32), dev), act)
+    q, d, s = act_host(m27q, act)
+    Y = torch.empty((M, rc), dtype=torch.float32, device=dev)
+    say("wide 2-byte base", type_name, rc, k)
+    m27q.matmul_q8(w, act, Y)
+    got = to_host(Y).astype(np.float64)
+    for m in (0, 17, M - 1):
+        want, nrm = ora.gemv_act(t, wb, rb, rc, q[m], d[m], s[m])
+        assert (np.abs(got[m] - want) <= int_dot_tol(nrm)).all(), m
