@@ -228,3 +228,29 @@ def test_c_caller_cpu(m27q):
     r = subprocess.run([C_CALLER, "--cpu"], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "abi_caller: ok" in r.stdout
+
+
+def test_packed_weight_arguments(m27q):
+    """The packed weight records and pointer arrays that the binding passes are
+    the ctypes ones, byte for byte; fields out of their range are wrapped as
+    ctypes wraps them (and then refused); a missing output is a NULL pointer."""
+    class T:
+        def __init__(self, p):
+            self.p = p
+
+        def data_ptr(self):
+            return self.p
+
+    ws = [m27q.Weight(T(FAKE + 256 * i), t, 20 + i, 7 + i, i % 2)
+          for i, t in enumerate((m27q.Q4_K, m27q.Q6_K, m27q.Q8_0, m27q.IQ4_XS))]
+    for w in ws:
+        assert m27q._weight(w) == bytes(w.desc())
+    assert m27q._weights(ws) == bytes((m27q.WeightDesc * 4)(*[w.desc() for w in ws]))
+    assert m27q._ptrs([T(1 << 40), None, T(3)], 3) == bytes((C.c_void_p * 3)(1 << 40, None, 3))
+    assert bytes(m27q._ptrs([T(16)], 2)) == bytes((C.c_void_p * 2)(16, None))
+    with pytest.raises(IndexError):
+        m27q._ptrs([T(1), T(2)], 1)
+    bad = m27q.Weight(T(FAKE), m27q.Q4_K, -1, 8, m27q.TILED)
+    L, y = m27q.lib(), (C.c_void_p * 1)(FAKE)
+    assert L.m27q_matvec(m27q._weight(bad), FAKE, FAKE, None, None, None) == 2
+    assert L.m27q_matvec_multi(1, m27q._weights([bad]), FAKE, y, None) == 2
