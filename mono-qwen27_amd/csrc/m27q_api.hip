@@ -94,8 +94,6 @@ ActView act_view(const void *xq, int M, int K) {
             (const uint32_t *)(b + m27q_act_s_offset(M, K))};
 }
 
-int wg_count(int rows) { return ((rows + kTileRows - 1) / kTileRows + kWavesPerWG - 1) / kWavesPerWG; }
-
 m27q_status hip_status(hipError_t e) { return e == hipSuccess ? M27Q_OK : M27Q_ERR_HIP; }
 
 m27q_status check_out_quant(const m27q_weight *w, const void *yq) {
@@ -400,9 +398,7 @@ M27Q_API m27q_status m27q_matvec_f32(const m27q_weight *w, const float *x, float
     p.res[0] = residual;
     p.rc[0] = (int)w->row_count;
     p.nmat = 1;
-    const int grid = wg_count((int)w->row_count);
-    p.wg_start[1] = grid;
-    return hip_status(launch_gemv_f32(w->ggml_type, (int)w->layout, p, grid, stream));
+    return hip_status(launch_gemv_f32(w->ggml_type, (int)w->layout, p, stream));
 }
 
 M27Q_API m27q_status m27q_matvec(const m27q_weight *w, const float *x, float *y, const float *residual, void *yq,

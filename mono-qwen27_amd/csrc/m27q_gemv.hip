@@ -25,8 +25,8 @@
 //   [w T / G, (w + 1) T / G), so one workgroup per CU carries an even share
 //   of a matrix whose tile count is not a multiple of the CU count.
 //
-// fp32-activation products (exact dequantization, fp32 accumulation) keep the
-// simpler one-wave-per-tile mapping: they are the fallback, not the hot path.
+// fp32-activation products (exact dequantization, fp32 accumulation) keep a
+// simpler mapping: a tile per wave, or per workgroup with K split over its waves.
 //
 // Replaces k_q4k_mv_q8_dp4a / k_q6k_mv_q8_dp4a / k_q80_mv_q8_dp4a
 // (exec:320-364, :631-645, :535-580), k_q5k_mv_q8 (exec:497-531),
@@ -344,14 +344,15 @@ struct TileSrc {
 };
 
 // acc += sum over units of T::dot_f32 with a two-stage load pipeline.
+// (units [ua, upr) here).
 template <class T, int LAYOUT, int kDepth, class A>
-__device__ __forceinline__ float stream_row_f32(const TileSrc<T, LAYOUT> &src, const A &act, int upr) {
+__device__ __forceinline__ float stream_row_f32(const TileSrc<T, LAYOUT> &src, const A &act, int ua, int upr) {
     typename T::Frag fa[kDepth], fb[kDepth];
     float acc = 0.f;
 #pragma unroll
     for (int k = 0; k < kDepth; ++k)
-        if (k < upr) fa[k] = src.load(k);
-    for (int u0 = 0; u0 < upr; u0 += 2 * kDepth) {
+        if (ua + k < upr) fa[k] = src.load(ua + k);
+    for (int u0 = ua; u0 < upr; u0 += 2 * kDepth) {
 #pragma unroll
         for (int k = 0; k < kDepth; ++k)
             if (u0 + kDepth + k < upr) fb[k] = src.load(u0 + kDepth + k);
@@ -368,9 +369,29 @@ __device__ __forceinline__ float stream_row_f32(const TileSrc<T, LAYOUT> &src, c
     return acc;
 }
 
-// One workgroup = 4 waves = 32 rows; x and its per-16 sums staged in LDS.
-template <class T, int LAYOUT>
-__global__ __launch_bounds__(256) void k_gemv_f32(GemvParams p) {
+// The sum of a row's K slices over the workgroup's KS waves, in wave order:
+// each wave's row sums (lanes c == 0 of row i) through LDS.  The result is in
+// the first 8 threads (row = thread).
+template <int KS>
+__device__ __forceinline__ float sum_slices(float *red, float acc, int wave, int i, int c) {
+    __syncthreads();  // red may overlay x
+    if (c == 0) red[wave * kTileRows + i] = acc;
+    __syncthreads();
+    float v = 0.f;
+    if (threadIdx.x < kTileRows) {
+        v = red[threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < KS; ++w) v += red[w * kTileRows + threadIdx.x];
+    }
+    return v;
+}
+
+// x and its per-16 sums staged in LDS.  KS = 1: 4 waves of one 8-row tile each.
+// KS = 8: the workgroup's 8 waves take slices of K of one tile: these products
+// are latency chains (a wave waits for its loads every two units), and few
+// tiles leave most SIMDs without a wave otherwise (f32_split).
+template <class T, int LAYOUT, int KS>
+__global__ __launch_bounds__(KS == 1 ? 256 : kWave *KS) void k_gemv_f32(GemvParams p) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int Kp = p.upr * T::kUnitElems;
     float *xf = (float *)smem;
@@ -390,33 +411,44 @@ __global__ __launch_bounds__(256) void k_gemv_f32(GemvParams p) {
     using LM = LaneMap<T, LAYOUT>;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = LM::row(lane), c = LM::chunk(lane);
     const int rc = p.rc[0];
-    const int tile = (int)blockIdx.x * kWavesPerWG + wave;
+    const int tile = KS == 1 ? (int)blockIdx.x * kWavesPerWG + wave : (int)blockIdx.x;
     const int ntiles = (rc + kTileRows - 1) / kTileRows;
     const int row = tile * kTileRows + i;
     const int row_ld = row < rc ? row : rc - 1;
     float acc = 0.f;
     if (tile < ntiles) {
         const TileSrc<T, LAYOUT> src(p.W[0], tile, row_ld, p.rb, p.upr, lane);
-        acc = stream_row_f32<T, LAYOUT, 2>(src, act, p.upr);
+        acc = KS == 1 ? stream_row_f32<T, LAYOUT, 2>(src, act, 0, p.upr)
+                      : stream_row_f32<T, LAYOUT, 2>(src, act, p.upr * wave / KS, p.upr * (wave + 1) / KS);
     }
     acc = LM::sum(acc);
-    if (c == 0 && tile < ntiles && row < rc) p.y[0][row] = acc + (p.res[0] ? p.res[0][row] : 0.f);
+    if constexpr (KS == 1) {
+        if (c == 0 && tile < ntiles && row < rc) p.y[0][row] = acc + (p.res[0] ? p.res[0][row] : 0.f);
+    } else {
+        const float v = sum_slices<KS>(xf, acc, wave, i, c);
+        const int r = tile * kTileRows + (int)threadIdx.x;
+        if (threadIdx.x < kTileRows && r < rc) p.y[0][r] = v + (p.res[0] ? p.res[0][r] : 0.f);
+    }
 }
 
 // F16 / F32 weights (GGUF rows of K elements): 8 lanes per row stride over
 // 16-byte chunks of the row; x is read through L1/L2 (these matrices are small:
 // the reference uses F16 for the 48 x 5120 ssm_beta / ssm_alpha, exec:2496-2497).
-template <bool HALF>
-__global__ __launch_bounds__(256) void k_gemv_dense(GemvParams p) {
+// One tile per workgroup, its KS waves striding over the row's chunks together:
+// F32 48 x 5120 4.5 us against 52.6 with a wave per tile, F16 2048 x 5120 6.3
+// against 28.7, F32 17408 x 5120 71.6 against 103.7.
+template <bool HALF, int KS>
+__global__ __launch_bounds__(kWave *KS) void k_gemv_dense(GemvParams p) {
+    __shared__ float red[KS * kTileRows];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane >> 3, c = lane & 7;
     const int rc = p.rc[0];
-    const int row = ((int)blockIdx.x * kWavesPerWG + wave) * kTileRows + i;
+    const int row = (int)blockIdx.x * kTileRows + i;
     const int K = p.K;
     constexpr int kPer = HALF ? 8 : 4;  // elements per 16-byte chunk
     float acc = 0.f;
     if (row < rc) {
         const uint8_t *rp = p.W[0] + (size_t)row * K * (HALF ? 2 : 4);
-        for (int k0 = c * kPer; k0 < K; k0 += kLanesPerRow * kPer) {
+        for (int k0 = (wave * kLanesPerRow + c) * kPer; k0 < K; k0 += KS * kLanesPerRow * kPer) {
             const uint4 w = ld_u128(rp + (size_t)k0 * (HALF ? 2 : 4));
             const float4 xa = *(const float4 *)(p.x + k0);
             if constexpr (HALF) {
@@ -431,8 +463,9 @@ __global__ __launch_bounds__(256) void k_gemv_dense(GemvParams p) {
             }
         }
     }
-    acc = sum8(acc);
-    if (c == 0 && row < rc) p.y[0][row] = acc + (p.res[0] ? p.res[0][row] : 0.f);
+    const float v = sum_slices<KS>(red, sum8(acc), wave, i, c);
+    const int r = (int)blockIdx.x * kTileRows + (int)threadIdx.x;
+    if (threadIdx.x < kTileRows && r < rc) p.y[0][r] = v + (p.res[0] ? p.res[0][r] : 0.f);
 }
 
 // ------------------------------------------------------------- launchers --
@@ -548,32 +581,47 @@ size_t gemv_f32_lds_bytes(uint32_t type, int upr) {
     return Kp * 4 + Kp / 4;
 }
 
+// Which quantized products split K over the 8 waves of a workgroup per 8-row
+// tile (the others keep a wave per tile): every workgroup stages x, so up to one
+// workgroup per CU (Q4_K 48 x 5120 4.2 us against 9.6, 2048 x 1024 3.2 against
+// 3.8), and up to three if the rows are long (6144 x 5120 9.5 against 11.7, but
+// 6144 x 1024 4.9 against 4.2 and 16384 x 5120 18.3 against 15.8).
+static bool f32_split(int tiles, int upr) { return tiles <= cu_count() || (tiles <= 3 * cu_count() && upr >= 16); }
+constexpr int kF32Slices = 8;
+
 template <class T, int LAYOUT>
-static hipError_t launch_f32_t(const GemvParams &p, int grid, hipStream_t s) {
+static hipError_t launch_f32_t(const GemvParams &p, hipStream_t s) {
     const size_t lds = gemv_f32_lds_bytes(T::kType, p.upr);
-    hipLaunchKernelGGL((k_gemv_f32<T, LAYOUT>), dim3(grid), dim3(256), lds, s, p);
+    const int tiles = (p.rc[0] + kTileRows - 1) / kTileRows;
+    static_assert(T::kUnitElems >= kF32Slices * kTileRows, "the slices' sums fit over x");
+    if (f32_split(tiles, p.upr))
+        hipLaunchKernelGGL((k_gemv_f32<T, LAYOUT, kF32Slices>), dim3(tiles), dim3(kWave * kF32Slices), lds, s, p);
+    else
+        hipLaunchKernelGGL((k_gemv_f32<T, LAYOUT, 1>), dim3((tiles + kWavesPerWG - 1) / kWavesPerWG), dim3(256), lds, s, p);
+    return hipGetLastError();
+}
+
+template <bool HALF>
+static hipError_t launch_dense(const GemvParams &p, hipStream_t s) {
+    hipLaunchKernelGGL((k_gemv_dense<HALF, kF32Slices>), dim3((p.rc[0] + kTileRows - 1) / kTileRows),
+                       dim3(kWave * kF32Slices), 0, s, p);
     return hipGetLastError();
 }
 
 template <class T>
-static hipError_t launch_f32_l(const GemvParams &p, int layout, int grid, hipStream_t s) {
-    return layout == M27Q_LAYOUT_TILED ? launch_f32_t<T, M27Q_LAYOUT_TILED>(p, grid, s)
-                                       : launch_f32_t<T, M27Q_LAYOUT_GGUF>(p, grid, s);
+static hipError_t launch_f32_l(const GemvParams &p, int layout, hipStream_t s) {
+    return layout == M27Q_LAYOUT_TILED ? launch_f32_t<T, M27Q_LAYOUT_TILED>(p, s) : launch_f32_t<T, M27Q_LAYOUT_GGUF>(p, s);
 }
 
-hipError_t launch_gemv_f32(uint32_t type, int layout, const GemvParams &p, int grid, hipStream_t s) {
+hipError_t launch_gemv_f32(uint32_t type, int layout, const GemvParams &p, hipStream_t s) {
     switch (type) {
-        case kQ4_K: return launch_f32_l<Q4K>(p, layout, grid, s);
-        case kQ5_K: return launch_f32_l<Q5K>(p, layout, grid, s);
-        case kQ6_K: return launch_f32_l<Q6K>(p, layout, grid, s);
-        case kQ8_0: return launch_f32_l<Q80>(p, layout, grid, s);
-        case kIQ4_XS: return launch_f32_l<IQ4XS>(p, layout, grid, s);
-        case kF16:
-            hipLaunchKernelGGL((k_gemv_dense<true>), dim3(grid), dim3(256), 0, s, p);
-            return hipGetLastError();
-        case kF32:
-            hipLaunchKernelGGL((k_gemv_dense<false>), dim3(grid), dim3(256), 0, s, p);
-            return hipGetLastError();
+        case kQ4_K: return launch_f32_l<Q4K>(p, layout, s);
+        case kQ5_K: return launch_f32_l<Q5K>(p, layout, s);
+        case kQ6_K: return launch_f32_l<Q6K>(p, layout, s);
+        case kQ8_0: return launch_f32_l<Q80>(p, layout, s);
+        case kIQ4_XS: return launch_f32_l<IQ4XS>(p, layout, s);
+        case kF16: return launch_dense<true>(p, s);
+        case kF32: return launch_dense<false>(p, s);
         default: return hipErrorInvalidValue;
     }
 }

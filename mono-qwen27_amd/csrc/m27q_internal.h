@@ -46,7 +46,7 @@ size_t gemv_q8_lds_bytes(uint32_t type, int upr, bool swiglu, int cfg);
 int gemv_q8_tiles_per_wg(int cfg);
 hipError_t launch_gemv_q8(uint32_t type, int layout, bool swiglu, int cfg, const GemvParams &p, hipStream_t s);
 size_t gemv_f32_lds_bytes(uint32_t type, int upr);
-hipError_t launch_gemv_f32(uint32_t type, int layout, const GemvParams &p, int grid, hipStream_t s);
+hipError_t launch_gemv_f32(uint32_t type, int layout, const GemvParams &p, hipStream_t s);
 
 hipError_t launch_quant_act(const float *x, const float *gate, long long n, int8_t *q, float *d, uint32_t *s,
                             hipStream_t st);

@@ -53,7 +53,8 @@
 //     87 us against 58), and the weights' 8-byte pieces of a line come in
 //     several loads, so they are temporal (non-temporal: down 90 us against 79,
 //     Q4_K at M = 17-48 5-11% slower);
-//   - 12 or 16 waves per workgroup (2-group steps) were slower at every size;
+//   - 12 or 16 waves per workgroup (2-group steps) were slower at every size, and
+//     two units of weights in flight 3-5% slower than one;
 //   - offsets kept in registers instead of computed per step: down 90 -> 78 us.
 //
 // No reference counterpart: the reference runs prefill one token at a time
@@ -835,7 +836,9 @@ hipError_t launch_wide_nt(MatmulMultiParams p, hipStream_t s) {
 template <class T, int LAYOUT>
 hipError_t launch_wide_m(const MatmulMultiParams &p, hipStream_t s) {
     switch ((p.M + 15) / 16) {
-        case 1: return launch_wide_nt<T, 1, LAYOUT>(p, s);
+        case 1:  // fewer than 17 rows: only for types the 16-token kernel does not take
+            if constexpr (!T::kF16 && LAYOUT == M27Q_LAYOUT_GGUF) return launch_wide_nt<T, 1, LAYOUT>(p, s);
+            else return hipErrorInvalidValue;
         case 2: return launch_wide_nt<T, 2, LAYOUT>(p, s);
         case 3: return launch_wide_nt<T, 3, LAYOUT>(p, s);
         case 4: return launch_wide_nt<T, 4, LAYOUT>(p, s);

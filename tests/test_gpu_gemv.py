@@ -457,3 +457,31 @@ def test_mixed_type_pair_ssm_shapes(m27q, ora, dev, layout):
             want, nrm = ora.gemv_act(w.type, wb, w.rb, rc, q[0], d[0], s[0])
             assert (np.abs(got.astype(np.float64) - want) <= int_dot_tol(nrm)).all(), (form, name)
             assert np.array_equal(got.view(np.uint32), to_host(y1).view(np.uint32)), (form, name)
+
+
+@pytest.mark.parametrize("type_name,rc,k,layout", [
+    ("Q4_K", 13, 256, 1), ("Q6_K", 7, 768, 0), ("Q8_0", 9, 160, 1), ("Q8_0", 9, 32, 0), ("IQ4_XS", 100, 2304, 1),
+    ("Q5_K", 1, 4608, 0), ("Q4_K", 2048, 256, 1), ("Q4_K", 2049, 256, 1), ("Q6_K", 6137, 4096, 1), ("Q6_K", 6145, 4096, 0), ("F16", 1, 8, 0), ("F16", 50, 1000, 0),
+    ("F32", 50, 516, 0), ("F32", 16385, 64, 0)])
+def test_matvec_f32_split(m27q, ora, dev, type_name, rc, k, layout):
+    """Exact-dequantization products with K split over a workgroup's waves:
+    fewer units (or 16-byte chunks) than waves, slices of unequal length,
+    partial tiles, and both sides of the line past which a wave takes a tile."""
+    import torch
+    t = getattr(m27q, type_name)
+    rb = k // m27q.BLOCK_ELEMS[t]
+    if type_name in ("F16", "F32"):
+        wb = ora.quantize(t, np.random.default_rng(2).standard_normal((rc, k)).astype(np.float32))
+    else:
+        wb = ora.synth_weights(t, rc, k, seed=11)
+    w = m27q.Weight.upload(wb.reshape(-1), t, rb, rc, layout, dev)
+    x = np.random.default_rng(8).standard_normal(k).astype(np.float32)
+    res = np.random.default_rng(9).standard_normal(rc).astype(np.float32)
+    y = torch.full((rc + 8,), 7.0, dtype=torch.float32, device=dev)
+    say("matvec_f32 split", type_name, rc, k, layout)
+    m27q.matvec_f32(w, to_dev(x, dev), y, residual=to_dev(res, dev))
+    got = to_host(y).astype(np.float64)
+    assert (got[rc:] == 7.0).all()
+    want = ora.gemv_f64(t, wb, rb, rc, x) + res
+    scale = np.abs(ora.dequant(t, wb, rb, rc)).astype(np.float64) @ np.abs(x).astype(np.float64) + np.abs(res)
+    assert (np.abs(got[:rc] - want) <= 1e-5 * scale).all()
