@@ -61,28 +61,30 @@ _SIGS = {
     "m27q_act_s_offset": (_SZ, [_I, _I]),
     "m27q_quant_act": (_I, [_P, _I, _I, _P, _P]),
     "m27q_quant_act_gated": (_I, [_P, _P, _I, _I, _P, _P]),
-    "m27q_matvec_q8": (_I, [_P, _P, _P, _P, _P, _P]),
-    "m27q_matvec_q8_multi": (_I, [_I, _P, _P, _P, _P]),
-    "m27q_matvec_multi": (_I, [_I, _P, _P, _P, _P]),
-    "m27q_ffn_swiglu": (_I, [_P, _P, _P, _P, _P, _P]),
-    "m27q_ffn_swiglu_q8": (_I, [_P, _P, _P, _P, _P, _P]),
-    "m27q_matvec_f32": (_I, [_P, _P, _P, _P, _P]),
-    "m27q_matvec": (_I, [_P, _P, _P, _P, _P, _P]),
-    "m27q_matmul_q8": (_I, [_P, _I, _P, _P, _P, _P]),
-    "m27q_matmul_q8_multi": (_I, [_I, _P, _I, _P, _P, _P]),
-    "m27q_dequant_rows": (_I, [_P, _I, _I, _P, _P]),
-    "m27q_embed_rows": (_I, [_P, _P, _I, _P, _P, _P]),
-    "m27q_embed_token": (_I, [_P, C.c_int32, _P, _P]),
+    "m27q_matvec_q8": (_I, [C.POINTER(WeightDesc), _P, _P, _P, _P, _P]),
+    "m27q_matvec_q8_multi": (_I, [_I, C.POINTER(WeightDesc), _P, C.POINTER(_P), _P]),
+    "m27q_matvec_multi": (_I, [_I, C.POINTER(WeightDesc), _P, C.POINTER(_P), _P]),
+    "m27q_ffn_swiglu": (_I, [C.POINTER(WeightDesc), C.POINTER(WeightDesc), _P, _P, _P, _P]),
+    "m27q_ffn_swiglu_q8": (_I, [C.POINTER(WeightDesc), C.POINTER(WeightDesc), _P, _P, _P, _P]),
+    "m27q_matvec_f32": (_I, [C.POINTER(WeightDesc), _P, _P, _P, _P]),
+    "m27q_matvec": (_I, [C.POINTER(WeightDesc), _P, _P, _P, _P, _P]),
+    "m27q_matmul_q8": (_I, [C.POINTER(WeightDesc), _I, _P, _P, _P, _P]),
+    "m27q_matmul_q8_multi": (_I, [_I, C.POINTER(WeightDesc), _I, _P, C.POINTER(_P), _P]),
+    "m27q_dequant_rows": (_I, [C.POINTER(WeightDesc), _I, _I, _P, _P]),
+    "m27q_embed_rows": (_I, [C.POINTER(WeightDesc), _P, _I, _P, _P, _P]),
+    "m27q_embed_token": (_I, [C.POINTER(WeightDesc), C.c_int32, _P, _P]),
     "m27q_topk_scratch_bytes": (_SZ, [_I, _I]),
     "m27q_topk": (_I, [_P, _I, _I, _P, _P, _P, _SZ, _P]),
     "m27q_topk_noalloc": (_I, [_P, _I, _I, _P, _P, _P]),
     "m27q_sample": (_I, [_P, _P, _I, C.c_float, C.c_float, C.c_float, _P, _P, _P]),
 }
 
-_lib = None
+_lib = _fast = None
 
 
 def lib() -> C.CDLL:
+    """The library, every entry point with the argument types of the header:
+    weights as WeightDesc, an array of them or a pointer to one."""
     global _lib
     if _lib is None:
         if not os.path.exists(LIB_PATH):
@@ -94,6 +96,26 @@ def lib() -> C.CDLL:
             f.argtypes = args
         _lib = L
     return _lib
+
+
+class _Calls:
+    """The entry points by name."""
+
+
+def _calls() -> _Calls:
+    """The entry points as the wrappers below call them: where lib() takes weight
+    records or arrays of pointers by type, these take any pointer (c_void_p), so
+    that the wrappers can pass packed bytes."""
+    global _fast
+    if _fast is None:
+        L, c = lib(), _Calls()
+        for name, (res, args) in _SIGS.items():
+            f = L[name]  # a function object of its own, not lib()'s
+            f.restype = res
+            f.argtypes = [_P if a in (C.POINTER(WeightDesc), C.POINTER(_P)) else a for a in args]
+            setattr(c, name, f)
+        _fast = c
+    return _fast
 
 
 def header_symbols() -> list[str]:
@@ -271,7 +293,7 @@ class Act:
 
 
 def quant_act(x, act: Act, gate=None, stream=None) -> None:
-    L = _lib or lib()
+    L = _fast or _calls()
     if gate is None:
         st = L.m27q_quant_act(_ptr(x), act.M, act.K, _ptr(act.buf), _stream(stream))
         if st:
@@ -283,82 +305,83 @@ def quant_act(x, act: Act, gate=None, stream=None) -> None:
 
 
 def matvec_q8(w: Weight, act: Act, y, residual=None, yq: Act | None = None, stream=None) -> None:
-    st = (_lib or lib()).m27q_matvec_q8(_weight(w), _ptr(act.buf), _ptr(y), _ptr(residual),
-                                        None if yq is None else _ptr(yq.buf), _stream(stream))
+    st = (_fast or _calls()).m27q_matvec_q8(_weight(w), _ptr(act.buf), _ptr(y), _ptr(residual),
+                                            None if yq is None else _ptr(yq.buf), _stream(stream))
     if st:
         check(st, "m27q_matvec_q8")
 
 
 def matvec_q8_multi(ws: list[Weight], act: Act, ys: list, stream=None) -> None:
-    st = (_lib or lib()).m27q_matvec_q8_multi(len(ws), _weights(ws), _ptr(act.buf), _ptrs(ys, len(ws)), _stream(stream))
+    st = (_fast or _calls()).m27q_matvec_q8_multi(len(ws), _weights(ws), _ptr(act.buf), _ptrs(ys, len(ws)),
+                                                  _stream(stream))
     if st:
         check(st, "m27q_matvec_q8_multi")
 
 
 def matvec_multi(ws: list[Weight], x, ys: list, stream=None) -> None:
     """fp32 activation x shared by up to 4 weights (quantized inside the kernel)."""
-    st = (_lib or lib()).m27q_matvec_multi(len(ws), _weights(ws), _ptr(x), _ptrs(ys, len(ws)), _stream(stream))
+    st = (_fast or _calls()).m27q_matvec_multi(len(ws), _weights(ws), _ptr(x), _ptrs(ys, len(ws)), _stream(stream))
     if st:
         check(st, "m27q_matvec_multi")
 
 
 def ffn_swiglu_q8(gate: Weight, up: Weight, act: Act, y, yq: Act | None = None, stream=None) -> None:
-    st = (_lib or lib()).m27q_ffn_swiglu_q8(_weight(gate), _weight(up), _ptr(act.buf), _ptr(y),
-                                            None if yq is None else _ptr(yq.buf), _stream(stream))
+    st = (_fast or _calls()).m27q_ffn_swiglu_q8(_weight(gate), _weight(up), _ptr(act.buf), _ptr(y),
+                                                None if yq is None else _ptr(yq.buf), _stream(stream))
     if st:
         check(st, "m27q_ffn_swiglu_q8")
 
 
 def ffn_swiglu(gate: Weight, up: Weight, x, y, yq: Act | None = None, stream=None) -> None:
     """fp32 activation x (quantized inside the kernel)."""
-    st = (_lib or lib()).m27q_ffn_swiglu(_weight(gate), _weight(up), _ptr(x), _ptr(y),
-                                         None if yq is None else _ptr(yq.buf), _stream(stream))
+    st = (_fast or _calls()).m27q_ffn_swiglu(_weight(gate), _weight(up), _ptr(x), _ptr(y),
+                                             None if yq is None else _ptr(yq.buf), _stream(stream))
     if st:
         check(st, "m27q_ffn_swiglu")
 
 
 def matvec_f32(w: Weight, x, y, residual=None, stream=None) -> None:
-    st = (_lib or lib()).m27q_matvec_f32(_weight(w), _ptr(x), _ptr(y), _ptr(residual), _stream(stream))
+    st = (_fast or _calls()).m27q_matvec_f32(_weight(w), _ptr(x), _ptr(y), _ptr(residual), _stream(stream))
     if st:
         check(st, "m27q_matvec_f32")
 
 
 def matvec(w: Weight, x, y, residual=None, yq: Act | None = None, stream=None) -> None:
     """fp32 activation x (quantized inside the kernel); F16/F32 weights take the fp32 path."""
-    st = (_lib or lib()).m27q_matvec(_weight(w), _ptr(x), _ptr(y), _ptr(residual),
-                                     None if yq is None else _ptr(yq.buf), _stream(stream))
+    st = (_fast or _calls()).m27q_matvec(_weight(w), _ptr(x), _ptr(y), _ptr(residual),
+                                         None if yq is None else _ptr(yq.buf), _stream(stream))
     if st:
         check(st, "m27q_matvec")
 
 
 def matmul_q8(w: Weight, act: Act, Y, residual=None, stream=None) -> None:
-    st = (_lib or lib()).m27q_matmul_q8(_weight(w), act.M, _ptr(act.buf), _ptr(Y), _ptr(residual),
-                                        _stream(stream))
+    st = (_fast or _calls()).m27q_matmul_q8(_weight(w), act.M, _ptr(act.buf), _ptr(Y), _ptr(residual),
+                                            _stream(stream))
     if st:
         check(st, "m27q_matmul_q8")
 
 
 def matmul_q8_multi(ws: list[Weight], act: Act, Ys: list, stream=None) -> None:
-    st = (_lib or lib()).m27q_matmul_q8_multi(len(ws), _weights(ws), act.M, _ptr(act.buf), _ptrs(Ys, len(ws)),
-                                              _stream(stream))
+    st = (_fast or _calls()).m27q_matmul_q8_multi(len(ws), _weights(ws), act.M, _ptr(act.buf), _ptrs(Ys, len(ws)),
+                                                  _stream(stream))
     if st:
         check(st, "m27q_matmul_q8_multi")
 
 
 def dequant_rows(w: Weight, row0: int, nrows: int, out, stream=None) -> None:
-    st = (_lib or lib()).m27q_dequant_rows(_weight(w), row0, nrows, _ptr(out), _stream(stream))
+    st = (_fast or _calls()).m27q_dequant_rows(_weight(w), row0, nrows, _ptr(out), _stream(stream))
     if st:
         check(st, "m27q_dequant_rows")
 
 
 def embed_rows(w: Weight, ids, out, bad=None, stream=None) -> None:
-    st = (_lib or lib()).m27q_embed_rows(_weight(w), _ptr(ids), ids.numel(), _ptr(out), _ptr(bad), _stream(stream))
+    st = (_fast or _calls()).m27q_embed_rows(_weight(w), _ptr(ids), ids.numel(), _ptr(out), _ptr(bad), _stream(stream))
     if st:
         check(st, "m27q_embed_rows")
 
 
 def embed_token(w: Weight, token_id: int, out, stream=None) -> None:
-    st = (_lib or lib()).m27q_embed_token(_weight(w), token_id, _ptr(out), _stream(stream))
+    st = (_fast or _calls()).m27q_embed_token(_weight(w), token_id, _ptr(out), _stream(stream))
     if st:
         check(st, "m27q_embed_token")
 
@@ -369,17 +392,17 @@ def topk_scratch_bytes(n: int, k: int) -> int:
 
 def sample(idx, val, k: int, temperature: float, min_p: float, top_p: float, u, token, stream=None) -> None:
     """token[0] <- the candidate sample() picks for the uniform u[0] (device tensors)."""
-    check((_lib or lib()).m27q_sample(_ptr(idx), _ptr(val), k, temperature, min_p, top_p, _ptr(u), _ptr(token),
-                            _stream(stream)), "m27q_sample")
+    check((_fast or _calls()).m27q_sample(_ptr(idx), _ptr(val), k, temperature, min_p, top_p, _ptr(u), _ptr(token),
+                                          _stream(stream)), "m27q_sample")
 
 
 def topk(logits, k: int, idx, val, scratch, stream=None) -> None:
     n = logits.numel()
-    check((_lib or lib()).m27q_topk(_ptr(logits), n, k, _ptr(idx), _ptr(val), _ptr(scratch),
-                          scratch.numel() * scratch.element_size(), _stream(stream)), "m27q_topk")
+    check((_fast or _calls()).m27q_topk(_ptr(logits), n, k, _ptr(idx), _ptr(val), _ptr(scratch),
+                                        scratch.numel() * scratch.element_size(), _stream(stream)), "m27q_topk")
 
 
 def topk_noalloc(logits, k: int, idx, val, stream=None) -> None:
     """m27q_topk on the library's static scratch (no scratch argument)."""
-    check((_lib or lib()).m27q_topk_noalloc(_ptr(logits), logits.numel(), k, _ptr(idx), _ptr(val), _stream(stream)),
-          "m27q_topk_noalloc")
+    check((_fast or _calls()).m27q_topk_noalloc(_ptr(logits), logits.numel(), k, _ptr(idx), _ptr(val),
+                                                _stream(stream)), "m27q_topk_noalloc")

@@ -254,3 +254,23 @@ def test_packed_weight_arguments(m27q):
     L, y = m27q.lib(), (C.c_void_p * 1)(FAKE)
     assert L.m27q_matvec(m27q._weight(bad), FAKE, FAKE, None, None, None) == 2
     assert L.m27q_matvec_multi(1, m27q._weights([bad]), FAKE, y, None) == 2
+
+
+def test_library_argument_types(m27q):
+    """lib() takes weights as a program builds them: a WeightDesc itself, a
+    pointer to one or an array of them; a packed record, an address or a pointer
+    to another type is an ArgumentError, before and after a wrapper has called
+    the same entry point."""
+    L, d, y = m27q.lib(), W(m27q, t=99), (C.c_void_p * 1)(FAKE)
+    for _ in range(2):
+        for w in (d, C.byref(d), C.pointer(d), (m27q.WeightDesc * 1)(d)):
+            assert L.m27q_matvec(w, FAKE, FAKE, None, None, None) == 3
+            assert L.m27q_matmul_q8(w, 4, FAKE, FAKE, None, None) == 3
+            assert L.m27q_embed_token(w, 0, FAKE, None) == 3
+            assert L.m27q_matvec_q8_multi(1, w, FAKE, y, None) == 3
+        for w in (bytes(d), FAKE, C.byref(C.c_int(0)), y):
+            with pytest.raises(C.ArgumentError):
+                L.m27q_matvec(w, FAKE, FAKE, None, None, None)
+            with pytest.raises(C.ArgumentError):
+                L.m27q_matvec_q8_multi(1, (m27q.WeightDesc * 1)(d), FAKE, bytes(y), None)
+        assert m27q._calls().m27q_matvec(bytes(d), FAKE, FAKE, None, None, None) == 3
