@@ -197,6 +197,16 @@ def _ptr(t) -> int | None:
 _raw_stream = _raw_device = None
 
 
+def _forget_raw_stream() -> None:
+    global _raw_stream
+    _raw_stream = None
+
+
+# A forked child of a process that has used the GPU must not use it: the child
+# goes through torch.cuda.current_stream() again, which raises there.
+os.register_at_fork(after_in_child=_forget_raw_stream)
+
+
 def _stream(stream) -> int:
     global _raw_stream, _raw_device
     if stream is not None:

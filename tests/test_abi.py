@@ -274,3 +274,29 @@ def test_library_argument_types(m27q):
             with pytest.raises(C.ArgumentError):
                 L.m27q_matvec_q8_multi(1, (m27q.WeightDesc * 1)(d), FAKE, bytes(y), None)
         assert m27q._calls().m27q_matvec(bytes(d), FAKE, FAKE, None, None, None) == 3
+
+
+def test_forked_child_asks_torch_for_the_stream(m27q, monkeypatch):
+    """The raw stream accessors serve the process that initialised torch.cuda: a
+    forked child goes through torch.cuda.current_stream(), which refuses there,
+    and the parent keeps the accessors."""
+    import torch
+
+    def refused():
+        raise RuntimeError("forked")
+
+    monkeypatch.setattr(m27q, "_raw_device", lambda: 0)
+    monkeypatch.setattr(m27q, "_raw_stream", lambda d: 1234)
+    monkeypatch.setattr(torch.cuda, "current_stream", refused)
+    assert m27q._stream(None) == 1234
+    pid = os.fork()
+    if pid == 0:
+        code = 1
+        try:
+            m27q._stream(None)
+        except RuntimeError:
+            code = 0
+        finally:
+            os._exit(code)
+    assert os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1]) == 0
+    assert m27q._stream(None) == 1234
