@@ -429,36 +429,37 @@ __global__ __launch_bounds__(kWave) void k_sample(const int32_t *__restrict__ id
                                                   const float *__restrict__ u, int32_t *__restrict__ token) {
     static_assert(kTopkMaxK == kWave, "one candidate per lane");
     const int lane = (int)threadIdx.x;
+    if (!(temperature > 0.f)) {  // the first index alone: nothing else need be there
+        if (lane == 0) *token = idx[0];
+        return;
+    }
     const bool in = lane < k;
     const int src = in ? lane : 0;
     const int id = idx[src];
     const float v = val[src], v0 = val[0], rnd = *u;
-    const int best = __builtin_amdgcn_readfirstlane(id);
-    int pick_id = best;
-    if (temperature > 0.f) {
-        const float a = (v - v0) / temperature;
-        float p = a >= -87.0f ? exp_cw(a) : (a < -87.0f ? 0.0f : a);
-        p = in ? p : 0.f;
-        float prefix;
-        const float sum = ordered_sum(p, k, lane, prefix);
-        if (sum > 0.f && isfinite(sum)) {
-            p /= sum;
-            // min_p: drop candidates below p_0 * min_p; p_0 itself always
-            // stays unless min_p > 1, and then the pick falls back to best.
-            const float thresh = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(p))) * min_p;
-            bool kept = in && !(p < thresh);
-            uint64_t m = __ballot(kept);
-            if (m) {
-                ordered_sum(kept ? p : 0.f, k, lane, prefix);
-                if (top_p < 1.f) {  // cut after the first candidate whose running sum reaches top_p
-                    const uint64_t reach = __ballot(kept && prefix >= top_p);
-                    if (reach) m &= (reach & (0ull - reach)) * 2 - 1;
-                }
-                const int last = 63 - __clzll((long long)m);
-                const float pick = rnd * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(prefix), last));
-                const uint64_t hit = __ballot(kept && pick <= prefix) & m;
-                pick_id = __builtin_amdgcn_readlane(id, hit ? __ffsll((long long)hit) - 1 : last);
+    int pick_id = __builtin_amdgcn_readfirstlane(id);
+    const float a = (v - v0) / temperature;
+    float p = a >= -87.0f ? exp_cw(a) : (a < -87.0f ? 0.0f : a);
+    p = in ? p : 0.f;
+    float prefix;
+    const float sum = ordered_sum(p, k, lane, prefix);
+    if (sum > 0.f && isfinite(sum)) {
+        p /= sum;
+        // min_p: drop candidates below p_0 * min_p; p_0 itself always
+        // stays unless min_p > 1, and then the pick falls back to the first.
+        const float thresh = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(p))) * min_p;
+        bool kept = in && !(p < thresh);
+        uint64_t m = __ballot(kept);
+        if (m) {
+            ordered_sum(kept ? p : 0.f, k, lane, prefix);
+            if (top_p < 1.f) {  // cut after the first candidate whose running sum reaches top_p
+                const uint64_t reach = __ballot(kept && prefix >= top_p);
+                if (reach) m &= (reach & (0ull - reach)) * 2 - 1;
             }
+            const int last = 63 - __clzll((long long)m);
+            const float pick = rnd * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(prefix), last));
+            const uint64_t hit = __ballot(kept && pick <= prefix) & m;
+            pick_id = __builtin_amdgcn_readlane(id, hit ? __ffsll((long long)hit) - 1 : last);
         }
     }
     if (lane == 0) *token = pick_id;

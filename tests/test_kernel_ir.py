@@ -1,0 +1,57 @@
+"""What the kernels' own LLVM IR shows without a GPU: which memory a path reads,
+and that accesses which must stay in order are ordered for the compiler.  The
+sources are compiled here with the library's flags (device pass, IR as text)."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "mono-qwen27_amd", "csrc")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+pytestmark = pytest.mark.skipif(not shutil.which(HIPCC), reason="needs hipcc")
+
+
+def kernel_blocks(tmp_path, source, kernel):
+    """{label: lines} of one kernel of `source`, the entry block first."""
+    ir = tmp_path / "kernel.ll"
+    subprocess.run([HIPCC, "-O3", "-std=c++17", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "-I", CSRC, "--offload-device-only", "-S", "-emit-llvm", str(source), "-o",
+                    str(ir)], check=True, capture_output=True, timeout=600)
+    body = re.search(r"^define [^\n]*@\w*" + kernel + r"\w*\(([^\n]*)\{\n(.*?)^\}", ir.read_text(), re.M | re.S).group(2)
+    blocks, label = {"": []}, ""
+    for line in body.splitlines():
+        m = re.match(r"(\d+):", line)
+        if m:
+            label = m.group(1)
+            blocks[label] = []
+        elif line.strip():
+            blocks[label].append(line.strip())
+    return blocks
+
+
+def test_greedy_sampling_reads_the_first_index_alone(tmp_path):
+    """temperature <= 0 gives idx[0]: the candidates behind it, their values and
+    u are not read (a greedy caller need not have filled them)."""
+    blocks = kernel_blocks(tmp_path, os.path.join(CSRC, "m27q_topk.hip"), "8k_sample")
+    hot, seen, todo, loads = {}, set(), [""], []  # arguments: %0 idx, %1 val, %2 k, %3 temperature, ...
+    while todo:
+        b = todo.pop()
+        if b in seen:
+            continue
+        seen.add(b)
+        for line in blocks[b]:
+            m = re.match(r"(%\d+) = fcmp .*\b(ogt|ugt|ole|ule) float %3, 0\.0", line)
+            if m:
+                hot[m.group(1)] = m.group(2) in ("ogt", "ugt")
+            if re.search(r"= load ", line):
+                loads.append(re.search(r"load \w+, ptr addrspace\(1\) (%\d+)", line).group(1))
+            m = re.match(r"br i1 (%\d+), label %(\d+), label %(\d+)", line)
+            if m:  # the branch on the temperature: the side of temperature <= 0 alone
+                todo += [m.group(2 + hot[m.group(1)])] if m.group(1) in hot else [m.group(2), m.group(3)]
+            elif line.startswith("br label"):
+                todo.append(re.match(r"br label %(\d+)", line).group(1))
+    assert hot and loads == ["%0"], loads
