@@ -55,3 +55,35 @@ def test_greedy_sampling_reads_the_first_index_alone(tmp_path):
             elif line.startswith("br label"):
                 todo.append(re.match(r"br label %(\d+)", line).group(1))
     assert hot and loads == ["%0"], loads
+
+
+@pytest.mark.parametrize("wt,nt,layout", [("WQ80", 1, 0), ("WQ4K<false>", 2, 1), ("WQ6K", 4, 0)])
+def test_one_wave_slices_order_their_lds_accesses(tmp_path, wt, nt, layout):
+    """Wide products with one wave per slice of K: lanes hand activations to each
+    other through LDS without a barrier, so on every path a fence must stand
+    between an LDS write and the next read, and between a read and the next
+    write; otherwise the compiler may swap two whose own-lane addresses differ."""
+    src = tmp_path / "few.hip"
+    src.write_text('#include "m27q_wide.h"\nnamespace m27q {\nhipError_t one(const MatmulMultiParams &p, hipStream_t s) '
+                   "{ return launch_wide_t<%s, %d, ShapeFew, %d>(p, 1, s); }\n}\n" % (wt, nt, layout))
+    blocks = kernel_blocks(tmp_path, src, "13k_matmul_wide")
+    state = {b: set() for b in blocks}  # the LDS accesses that may be the last ones at a block's entry
+    state[""] = {""}
+    todo, accesses, swaps = [""], 0, []
+    while todo:
+        b = todo.pop()
+        now = set(state[b])
+        for line in blocks[b]:
+            if line.startswith("fence "):
+                now = {""}
+            elif "addrspace(3)" in line and re.match(r"(store|%\d+ = load) ", line):
+                kind = "store" if line.startswith("store") else "load"
+                accesses += 1
+                if now - {"", kind}:
+                    swaps.append((b, line))
+                now = {kind}
+        for t in re.findall(r"label %(\d+)", blocks[b][-1] if blocks[b][-1].startswith("br ") else ""):
+            if not now <= state[t]:
+                state[t] |= now
+                todo.append(t)
+    assert accesses > 20 and not swaps, swaps[:4]
