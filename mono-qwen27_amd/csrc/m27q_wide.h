@@ -14,10 +14,14 @@
 //     <= 1953; Q6_K's up to 4096 as an exact sum of two fp16 values), the int8
 //     codes are exact in fp16, and the fp32 MFMA accumulator holds the group's
 //     integer sum exactly (below 2^24).  What is left per (row, token, group)
-//     is one FMA with dx; d (and dmin) follow once per 256 weights;
+//     is one FMA with dx; d (and dmin) follow once per 256 weights.  Q4_K and
+//     Q5_K keep all of this 2^-10 down until the final sum, so that dx times a
+//     group's sum does not overflow where the result does not (results below
+//     2^-116 are sums of multiples of 2^-139 for it);
 //   - Q4_K / Q5_K's min term, sum_j m_j (dx_j sum(codes_j)), is one bf16 MFMA
 //     per tile and block: m_j is exact in bf16, and the fp32 token factor is
-//     split into three bf16 values that add up to it exactly;
+//     split into three bf16 values that add up to it exactly (two of them kept
+//     2^7 and 2^14 up against m_j as much down, for the smallest factors);
 //   - Q8_0 (a scale per 32 weights and row) and IQ4_XS (12-bit products) stay
 //     on int8 MFMA with the scales in fp32 afterwards.
 //
@@ -77,6 +81,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 
+constexpr int kMinStep = 7;  // powers of two between the parts of a min term's token factor
 constexpr uint32_t kH1024 = 0x64006400u;  // (1024, 1024) in fp16: or-ing an integer below 1024 in adds it
 
 __device__ __forceinline__ h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
@@ -176,16 +181,20 @@ struct WQ4K {
             }
         }
     }
-    // sc q of group G: 1024 + q (even groups; 1024 + 16 q for the high nibbles
-    // of odd ones) from one mask, then one FMA: (1024 + q) sc - 1024 sc, or
-    // with sc / 16; every intermediate is exact in fp16.
+    // 2^-10 sc q of group G: 1024 + q (even groups; 1024 + 16 q for the high
+    // nibbles of odd ones) from one mask, then one FMA: (1024 + q) s - 1024 s
+    // with s = 2^-10 sc, or 2^-14 sc; every intermediate is exact in fp16.  The
+    // 2^-10 (kDown; the final sum takes it back) keeps dx times the group's sum
+    // within fp32 wherever the 16-token kernel's, which applies sc later, is:
+    // without it rows of magnitude 1e34 to 1e36 came out infinite.
+    static constexpr int kDown = 10;
     template <int G, int LAYOUT>
     __device__ static AOp<false> operand(const Reg &r, int, uint32_t, const Cst &cst) {
         constexpr bool odd = G & 1;
         const uint32_t scw = G < 4 ? (r.h.y & 0x3f3f3f3fu) : ((r.h.w & 0x0f0f0f0fu) | ((r.h.y >> 2) & 0x30303030u));
         constexpr uint32_t sel = 0x04000400u | (uint32_t)(G & 3) | ((uint32_t)(G & 3) << 16);
         const h2 t = as_h2(__builtin_amdgcn_perm(0x64646464u, scw, sel));  // 1024 + sc
-        const h2 s = odd ? pk_fma(t, splat(0.0625f), splat(-64.f)) : t - splat(1024.f);
+        const h2 s = odd ? pk_fma(t, splat(0x1p-14f), splat(-0x1p-4f)) : pk_fma(t, splat(0x1p-10f), splat(-1.f));
         const h2 n = s * splat(-1024.f);
         const uint32_t m = odd ? cst.hi : cst.lo;
         uint32_t w[4];
@@ -205,9 +214,13 @@ struct WQ4K {
         }
         return {make_h8(w[0], w[1], w[2], w[3])};
     }
-    // The min term's weight operand: m_0 .. m_7 of row c in bf16 in lane
-    // quarters 0-2 (against the three parts of the token factors), 0 in quarter 3.
+    // The min term's weight operand: 2^-(10 + 7 q) m_0 .. m_7 of row c in bf16
+    // in lane quarters q = 0-2 (against the three parts of the token factors,
+    // the second and third of which are kept 2^7 and 2^14 up), 0 in quarter 3.
+    // The power of two is taken off the exponents (m = 0 saturates at 0).
     __device__ static b8 min_operand(const Reg &r, int q) {
+        typedef uint16_t s2 __attribute__((ext_vector_type(2)));
+        const s2 down = (s2)(uint16_t)((kDown + kMinStep * q) << 7);
         const uint32_t on = q < 3 ? ~0u : 0u;
         const uint32_t m0 = r.h.z & (0x3f3f3f3fu & on);
         const uint32_t m1 = (((r.h.w >> 4) & 0x0f0f0f0fu) | ((r.h.z >> 2) & 0x30303030u)) & on;
@@ -216,7 +229,8 @@ struct WQ4K {
         for (int k = 0; k < 4; ++k) {
             const uint32_t m = k < 2 ? m0 : m1;
             const int e = 2 * (k & 1);
-            w[k] = __builtin_amdgcn_perm(__float_as_uint(ubyte(m, e + 1)), __float_as_uint(ubyte(m, e)), 0x07060302u);
+            const uint32_t b = __builtin_amdgcn_perm(__float_as_uint(ubyte(m, e + 1)), __float_as_uint(ubyte(m, e)), 0x07060302u);
+            w[k] = __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(s2, b), down));
         }
         return __builtin_bit_cast(b8, u4{w[0], w[1], w[2], w[3]});
     }
@@ -228,6 +242,7 @@ struct WQ4K {
 // .., bits 2 rr of qh bytes 32 h .., scale 8 h + 2 rr + (position / 16).
 struct WQ6K {
     static constexpr bool kF16 = true, kMin = false, kTwo = true, kInterleave = false, kRagged = false;
+    static constexpr int kDown = 0;
     static constexpr int kUnitBytes = kQ6KUnit, kBlockBytes = kQ6KBytes;
     struct Reg {
         u2 ql[4], qh[2];
@@ -304,6 +319,7 @@ struct WQ6K {
 // A unit here is 8 blocks (two TILED units).
 struct WQ80 {
     static constexpr bool kF16 = false, kMin = false, kTwo = false, kInterleave = false, kRagged = true;
+    static constexpr int kDown = 0;
     static constexpr int kUnitBytes = kQ80Unit, kBlockBytes = kQ80Bytes;
     struct Reg {
         u2 q[8];
@@ -342,6 +358,7 @@ struct WQ80 {
 // ---------------------------------------------------------------- IQ4_XS --
 struct WIQ4XS {
     static constexpr bool kF16 = false, kMin = false, kTwo = false, kInterleave = true, kRagged = false;
+    static constexpr int kDown = 0;
     static constexpr int kUnitBytes = kIQ4XSUnit, kBlockBytes = kIQ4XSBytes;
     struct Reg {
         uint32_t q[8];  // qs bytes 4 q .. + 4 of each group
@@ -571,12 +588,14 @@ __global__ __launch_bounds__(kWave *SH::W, SH::W / 4) void k_matmul_wide(MatmulM
                 const float d = __uint_as_float(rd[R][n]);
                 *(float *)(dT + sdst[n]) = d;
                 if constexpr (T::kMin) {
-                    // dx sum(codes) as three bf16 values (each the top half of
-                    // what is left; the remainders are exact)
+                    // dx sum(codes) as three bf16 values: each the top half of
+                    // what is left, and the rest (below 2^-7 of it, exact) moved
+                    // 2^7 up, so that the smallest factors keep their last bits
                     const int sum = (int)(int16_t)(rx[R][n] & 0xffffu) + (int)(int16_t)(rx[R][n] >> 16);
                     const float a = d * (float)sum;
-                    const float r1 = a - __uint_as_float(__float_as_uint(a) & 0xffff0000u);
-                    const float r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
+                    constexpr float up = (float)(1 << kMinStep);
+                    const float r1 = (a - __uint_as_float(__float_as_uint(a) & 0xffff0000u)) * up;
+                    const float r2 = (r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u)) * up;
                     uint8_t *ax = sl + C::oAux + ubuf * C::kAux + xdst[n] + 2 * decltype(st)::value * GS;
                     *(uint16_t *)ax = (uint16_t)(__float_as_uint(a) >> 16);
                     *(uint16_t *)(ax + 16 * 16) = (uint16_t)(__float_as_uint(r1) >> 16);
@@ -815,7 +834,7 @@ __global__ __launch_bounds__(kWave *SH::W, SH::W / 4) void k_matmul_wide(MatmulM
             const float *r = p.res[mi] ? p.res[mi] + o : nullptr;
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (row + e < rc) y[e] = v[e] + (r ? r[e] : 0.f);
+                if (row + e < rc) y[e] = v[e] * (float)(1 << T::kDown) + (r ? r[e] : 0.f);
         }
     }
 }

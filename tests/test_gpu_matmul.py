@@ -300,3 +300,49 @@ def test_wide_two_byte_aligned_base(m27q, ora, dev, type_name, rc, k):
     for m in (0, 17, M - 1):
         want, nrm = ora.gemv_act(t, wb, rb, rc, q[m], d[m], s[m])
         assert (np.abs(got[m] - want) <= int_dot_tol(nrm)).all(), m
+
+
+@pytest.mark.parametrize("type_name,rc,M,layout,big", [
+    ("Q4_K", 100, 20, 1, 1e36), ("Q4_K", 4200, 40, 0, 1e36), ("Q5_K", 100, 33, 0, 1e36), ("Q5_K", 4200, 64, 1, 1e36),
+    ("Q6_K", 4200, 40, 1, 1e33), ("Q6_K", 100, 20, 0, 1e33), ("Q8_0", 4200, 40, 1, 1e37), ("IQ4_XS", 4200, 40, 1, 1e37)])
+def test_wide_extreme_rows(m27q, ora, dev, type_name, rc, M, layout, big):
+    """One activation row at the ends of the float range among ordinary ones:
+    a row of magnitude `big` (the largest power of ten whose sums every other
+    kernel keeps finite) and one of 1e-36 against the oracle, NaN values (code
+    0) likewise, and a row with an infinity (NaN); the other rows' bits stay."""
+    import torch
+    t, k, r = getattr(m27q, type_name), 512, 7
+    rb = k // m27q.BLOCK_ELEMS[t]
+    wb = ora.synth_weights(t, rc, k, seed=3)
+    w = m27q.Weight.upload(wb.reshape(-1), t, rb, rc, layout, dev)
+    X0 = np.random.default_rng(5).standard_normal((M, k)).astype(np.float32)
+
+    def product(X):
+        act = m27q.Act(M, k, dev)
+        m27q.quant_act(to_dev(X, dev), act)
+        Y = torch.empty((M, rc), dtype=torch.float32, device=dev)
+        m27q.matmul_q8(w, act, Y)
+        return to_host(Y), [a[r] for a in act_host(m27q, act)]
+
+    base, _ = product(X0)
+    for name in ("big", "small", "nan", "inf"):
+        X = X0.copy()
+        if name == "nan":
+            X[r, 3] = np.nan
+            X[r, 32:64] = np.nan
+        elif name == "inf":
+            X[r, 3] = -np.inf
+        else:
+            X[r] = (X[r].astype(np.float64) * (big if name == "big" else 1e-36)).astype(np.float32)
+        say("wide extreme", type_name, rc, M, layout, name)
+        Y, (q, d, s) = product(X)
+        assert np.array_equal(np.delete(Y, r, 0).view(np.uint32), np.delete(base, r, 0).view(np.uint32)), name
+        if name == "inf":
+            assert np.isnan(Y[r]).all()
+            continue
+        want, nrm = ora.gemv_act(t, wb, rb, rc, q, d, s)
+        # 1e-36: every product and sum is also rounded to a multiple of 2^-149 (of
+        # Q4_K / Q5_K's sums, kept 2^-10 down, 2^-139); Q8_0 / IQ4_XS round the
+        # scales' product so before it meets a 12-bit sum
+        tiny = k * 2.0 ** -149 * (2.0 ** 12 if type_name in ("Q8_0", "IQ4_XS") else 1024.0)
+        assert (np.abs(Y[r].astype(np.float64) - want) <= 1e-6 * nrm + (tiny if name == "small" else 0)).all(), name
