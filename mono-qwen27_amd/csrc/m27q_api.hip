@@ -210,9 +210,10 @@ m27q_status gemv_impl(int n, const m27q_weight *ws, const void *xq, const float 
 // against 20.1 on MFMA).
 // GGUF-layout weights take the same few-token kernel (with temporal loads);
 // from M = 3, GGUF-layout Q4_K / Q5_K / Q6_K take the MFMA kernel (staged from
-// the row blocks), GGUF-layout Q8_0 and IQ4_XS one launch per matrix of the
-// VALU kernel (m27q_matmul.hip).  More rows take the wide kernel (m27q_wide.h,
-// matmul_wide_wins).
+// the row blocks), GGUF-layout Q8_0 and IQ4_XS one launch per matrix and 16
+// rows of the VALU kernel (m27q_matmul.hip).  Where matmul_wide_wins says so
+// (m27q_route.h: from 17 rows, GGUF Q8_0 / IQ4_XS from 5), the wide kernel
+// (m27q_wide.h) takes their place.
 constexpr int kMtMaxM = 2;
 constexpr size_t kMtLdsBudget = 80 * 1024;  // two workgroups per CU
 
@@ -240,8 +241,8 @@ m27q_status matmul_multi_impl(int n, const m27q_weight *ws, int M, const void *x
                      matmul_mt_lds_bytes(type, p.upr) <= kMtLdsBudget;
     long long sets = 0;
     for (int i = 0; i < n; ++i) sets += ((long long)ws[i].row_count + 15) / 16;
-    const bool wide = !few && lds_limit() >= kWideLds && matmul_wide_wins(type, layout, sets, M, cu_count());
-    if (!few && !wide && !matmul_mfma_takes(type, layout)) {  // GGUF Q8_0 / IQ4_XS of a few rows
+    const bool wide = !few && lds_limit() >= kWideLds && matmul_wide_wins(type, layout, sets, p.K, M, cu_count());
+    if (!few && !wide && !matmul_mfma_takes(type, layout)) {  // GGUF Q8_0 / IQ4_XS
         if (dry) return M27Q_OK;
         for (int i = 0; i < n; ++i) {
             MatmulParams q{};

@@ -9,6 +9,7 @@
 #include "../../include/m27q.h"
 #include "m27q_gemv_cfg.h"
 #include "m27q_layout.h"
+#include "m27q_route.h"
 
 namespace m27q {
 
@@ -114,39 +115,17 @@ hipError_t launch_matmul_mt(uint32_t type, int layout, const MatmulMultiParams &
 // GGUF-layout Q4_K / Q5_K / Q6_K (matmul_mfma_takes), any M (16 tokens per
 // launch).
 size_t matmul_mfma_lds_bytes(uint32_t type);
-bool matmul_mfma_takes(uint32_t type, int layout);
 // Whether its weight operands go straight into registers (TILED Q4_K / Q5_K).
 bool matmul_mfma_direct(uint32_t type, int layout);
 // Up to 64 tokens in one pass over the weights (m27q_wide.h), every type and
-// layout; a weight of any size (its descriptors cover 16 rows each).
+// layout (which products take it: matmul_wide_wins); a weight of any size (its
+// descriptors cover 16 rows each).
 constexpr size_t kWideLds = 160 * 1024;  // LDS its largest launch shapes take
 hipError_t launch_wide_q4k(int layout, const MatmulMultiParams &p, hipStream_t s);
 hipError_t launch_wide_q5k(int layout, const MatmulMultiParams &p, hipStream_t s);
 hipError_t launch_wide_q6k(int layout, const MatmulMultiParams &p, hipStream_t s);
 hipError_t launch_wide_q80(int layout, const MatmulMultiParams &p, hipStream_t s);
 hipError_t launch_wide_iq4xs(int layout, const MatmulMultiParams &p, hipStream_t s);
-// Whether the wide kernel is the faster one, for `sets` 16-row sets on `cus` CUs.
-// GGUF-layout Q8_0 / IQ4_XS (otherwise the VALU kernel): from 9 rows on always
-// (Q8_0 6144 x 6144 at M = 9 36.0 us against 85.4), from 5 with at most one set
-// per CU (1024 x 5120 15.8 against 38.4); at M = 3 / 5 on 17408 x 5120 IQ4_XS
-// the VALU kernel takes 21.9 / 29.5 us against 34.3.
-// The other types and layout have launches of 16 tokens of the MFMA kernel.
-// Past 32 tokens (three or four launches against one) the wide kernel always
-// wins: Q4_K 17408 x 5120 at M = 64 34.7 us against 81.9, Q6_K 5120 x 17408
-// 65.0 against 103.0.  At 17 to 32 it replaces two launches, and its fixed split
-// of two sets per workgroup between one and two sets per CU leaves CUs idle:
-// 320 sets (5120 x 17408) draw or lose on every type (Q6_K 48.3 against 45.3 us
-// at M = 17), GGUF Q6_K and IQ4_XS up to two sets per CU (IQ4_XS 6144 x 6144
-// 21.9 against 19.6); with one set per CU or fewer, more than two, or on the
-// other types from 1.5 on it wins (Q4_K 8192 x 5120 14.5 against 15.3, Q6_K
-// 8192 x 5120 18.0 against 21.5, Q4_K 17408 x 5120 23.4 against 34.2).
-inline bool matmul_wide_wins(uint32_t type, int layout, long long sets, int M, int cus) {
-    const bool gguf = layout == M27Q_LAYOUT_GGUF;
-    if (!matmul_mfma_takes(type, layout)) return M > 8 || (M > 4 && sets <= cus);
-    if (M <= 16) return false;
-    if (M > 32 || sets <= cus || sets > 2 * cus) return true;
-    return 2 * sets >= 3 * cus && type != kIQ4_XS && !(gguf && type == kQ6_K);
-}
 inline hipError_t launch_matmul_wide(uint32_t type, int layout, const MatmulMultiParams &p, hipStream_t s) {
     switch (type) {
         case kQ4_K: return launch_wide_q4k(layout, p, s);

@@ -1,8 +1,8 @@
-// m27q_matmul.hip -- products of up to 8 rows on GGUF-layout Q8_0 / IQ4_XS weights
-// (matmul_wide_wins): Y[M][N] = X[M][K] W[N][K]^T.
+// m27q_matmul.hip -- small-M products on GGUF-layout Q8_0 / IQ4_XS weights that
+// the wide kernel does not take (matmul_wide_wins): Y[M][N] = X[M][K] W[N][K]^T.
 //
 // Same wavefront tiling as the M = 1 GEMV (8 rows per wave, 16-byte weight
-// loads); the weights are read once per group of up to 8 activation rows and
+// loads); the weights are read once per group of up to 16 activation rows and
 // each lane keeps one accumulator per row.  Activations are staged in LDS per
 // K-chunk of 4 units for all rows of the group, so LDS stays small at any K.
 // No reference counterpart: the reference feeds prefill one token at a time
@@ -99,11 +99,12 @@ static hipError_t launch_mt(const MatmulParams &p, int m0, hipStream_t s) {
 template <class T>
 static hipError_t launch_m(const MatmulParams &p, hipStream_t s) {
     constexpr int L = M27Q_LAYOUT_GGUF;
-    for (int m0 = 0; m0 < p.M; m0 += 8) {
+    for (int m0 = 0; m0 < p.M; m0 += 16) {
         const int left = p.M - m0;
         const hipError_t e = left <= 2   ? launch_mt<T, L, 2>(p, m0, s)
                              : left <= 4 ? launch_mt<T, L, 4>(p, m0, s)
-                                         : launch_mt<T, L, 8>(p, m0, s);
+                             : left <= 8 ? launch_mt<T, L, 8>(p, m0, s)
+                                         : launch_mt<T, L, 16>(p, m0, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

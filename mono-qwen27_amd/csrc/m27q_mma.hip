@@ -1419,10 +1419,6 @@ size_t matmul_mfma_lds_bytes(uint32_t type) {
     }
 }
 
-bool matmul_mfma_takes(uint32_t type, int layout) {
-    return layout == M27Q_LAYOUT_TILED || type == kQ4_K || type == kQ5_K || type == kQ6_K;
-}
-
 bool matmul_mfma_direct(uint32_t type, int layout) {
     return layout == M27Q_LAYOUT_TILED && (type == kQ4_K || type == kQ5_K);
 }

@@ -346,3 +346,29 @@ def test_wide_extreme_rows(m27q, ora, dev, type_name, rc, M, layout, big):
         # scales' product so before it meets a 12-bit sum
         tiny = k * 2.0 ** -149 * (2.0 ** 12 if type_name in ("Q8_0", "IQ4_XS") else 1024.0)
         assert (np.abs(Y[r].astype(np.float64) - want) <= 1e-6 * nrm + (tiny if name == "small" else 0)).all(), name
+
+
+@pytest.mark.parametrize("type_name,rc,k,M", [
+    ("Q8_0", 12401, 160, 9), ("Q8_0", 20003, 992, 16), ("IQ4_XS", 12401, 256, 16), ("IQ4_XS", 13000, 768, 11),
+    ("Q8_0", 82001, 64, 17), ("Q8_0", 82001, 32, 24), ("IQ4_XS", 82001, 256, 20)])
+def test_gguf_valu_16_rows(m27q, ora, dev, type_name, rc, k, M):
+    """GGUF Q8_0 / IQ4_XS on many sets: launches of up to 16 rows of the VALU
+    kernel (one or two units of K, ragged Q8_0 units, a second launch of 1, 4
+    and 8 rows), every row with a residual against the oracle."""
+    import torch
+    t = getattr(m27q, type_name)
+    rb = k // m27q.BLOCK_ELEMS[t]
+    wb = ora.synth_weights(t, rc, k, seed=43)
+    w = m27q.Weight.upload(wb.reshape(-1), t, rb, rc, m27q.GGUF, dev)
+    act = m27q.Act(M, k, dev)
+    m27q.quant_act(to_dev(np.random.default_rng(M).standard_normal((M, k)).astype(np.float32), dev), act)
+    res = np.random.default_rng(M + 1).standard_normal((M, rc)).astype(np.float32)
+    Y = torch.full((M + 1, rc), 7.0, dtype=torch.float32, device=dev)
+    say("gguf valu", type_name, rc, k, M)
+    m27q.matmul_q8(w, act, Y[:M], residual=to_dev(res, dev))
+    got = to_host(Y).astype(np.float64)
+    assert (got[M] == 7.0).all()
+    q, d, s = act_host(m27q, act)
+    for m in range(M):
+        want, nrm = ora.gemv_act(t, wb, rb, rc, q[m], d[m], s[m])
+        assert (np.abs(got[m] - res[m] - want) <= int_dot_tol(nrm) + 1e-6 * np.abs(res[m])).all(), m
