@@ -434,21 +434,22 @@ __global__ __launch_bounds__(KS == 1 ? 256 : kWave *KS) void k_gemv_f32(GemvPara
 // F16 / F32 weights (GGUF rows of K elements): 8 lanes per row stride over
 // 16-byte chunks of the row; x is read through L1/L2 (these matrices are small:
 // the reference uses F16 for the 48 x 5120 ssm_beta / ssm_alpha, exec:2496-2497).
-// One tile per workgroup, its KS waves striding over the row's chunks together:
-// F32 48 x 5120 4.5 us against 52.6 with a wave per tile, F16 2048 x 5120 6.3
-// against 28.7, F32 17408 x 5120 71.6 against 103.7.
+// KS = 1: 4 waves of one tile each.  KS = 8: one tile per workgroup, its waves
+// striding over the row's chunks together, for rows of more than kDenseRow
+// bytes: F32 48 x 5120 4.5 us against 52.6 with a wave per tile, F16 2048 x 5120
+// 6.3 against 28.7, F32 17408 x 5120 71.6 against 103.7.
 template <bool HALF, int KS>
-__global__ __launch_bounds__(kWave *KS) void k_gemv_dense(GemvParams p) {
+__global__ __launch_bounds__(KS == 1 ? 256 : kWave *KS) void k_gemv_dense(GemvParams p) {
     __shared__ float red[KS * kTileRows];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane >> 3, c = lane & 7;
     const int rc = p.rc[0];
-    const int row = (int)blockIdx.x * kTileRows + i;
+    const int row = (KS == 1 ? (int)blockIdx.x * kWavesPerWG + wave : (int)blockIdx.x) * kTileRows + i;
     const int K = p.K;
     constexpr int kPer = HALF ? 8 : 4;  // elements per 16-byte chunk
     float acc = 0.f;
     if (row < rc) {
         const uint8_t *rp = p.W[0] + (size_t)row * K * (HALF ? 2 : 4);
-        for (int k0 = (wave * kLanesPerRow + c) * kPer; k0 < K; k0 += KS * kLanesPerRow * kPer) {
+        for (int k0 = ((KS == 1 ? 0 : wave) * kLanesPerRow + c) * kPer; k0 < K; k0 += KS * kLanesPerRow * kPer) {
             const uint4 w = ld_u128(rp + (size_t)k0 * (HALF ? 2 : 4));
             const float4 xa = *(const float4 *)(p.x + k0);
             if constexpr (HALF) {
@@ -463,9 +464,14 @@ __global__ __launch_bounds__(kWave *KS) void k_gemv_dense(GemvParams p) {
             }
         }
     }
-    const float v = sum_slices<KS>(red, sum8(acc), wave, i, c);
-    const int r = (int)blockIdx.x * kTileRows + (int)threadIdx.x;
-    if (threadIdx.x < kTileRows && r < rc) p.y[0][r] = v + (p.res[0] ? p.res[0][r] : 0.f);
+    acc = sum8(acc);
+    if constexpr (KS == 1) {
+        if (c == 0 && row < rc) p.y[0][row] = acc + (p.res[0] ? p.res[0][row] : 0.f);
+    } else {
+        const float v = sum_slices<KS>(red, acc, wave, i, c);
+        const int r = (int)blockIdx.x * kTileRows + (int)threadIdx.x;
+        if (threadIdx.x < kTileRows && r < rc) p.y[0][r] = v + (p.res[0] ? p.res[0][r] : 0.f);
+    }
 }
 
 // ------------------------------------------------------------- launchers --
@@ -585,9 +591,16 @@ size_t gemv_f32_lds_bytes(uint32_t type, int upr) {
 // tile (the others keep a wave per tile): every workgroup stages x, so up to one
 // workgroup per CU (Q4_K 48 x 5120 4.2 us against 9.6, 2048 x 1024 3.2 against
 // 3.8), and up to three if the rows are long (6144 x 5120 9.5 against 11.7, but
-// 6144 x 1024 4.9 against 4.2 and 16384 x 5120 18.3 against 15.8).
-static bool f32_split(int tiles, int upr) { return tiles <= cu_count() || (tiles <= 3 * cu_count() && upr >= 16); }
+// 6144 x 1024 4.9 against 4.2 and 16384 x 5120 18.3 against 15.8).  Rows of one or
+// two units leave most waves without work (Q4_K 2048 x 256 3.4 against 3.1).
+static bool f32_split(int tiles, int upr) {
+    return upr > 2 && (tiles <= cu_count() || (tiles <= 3 * cu_count() && upr >= 16));
+}
 constexpr int kF32Slices = 8;
+// F16 / F32 rows of up to this many bytes keep a wave per tile: the 64 lanes of
+// the split have at most one 16-byte chunk each (F16 200000 x 64 22.3 us against
+// 7.1, F32 50000 x 128 8.3 against 6.3; F16 50000 x 512 1.2x faster split).
+constexpr size_t kDenseRow = 512;
 
 template <class T, int LAYOUT>
 static hipError_t launch_f32_t(const GemvParams &p, hipStream_t s) {
@@ -603,8 +616,11 @@ static hipError_t launch_f32_t(const GemvParams &p, hipStream_t s) {
 
 template <bool HALF>
 static hipError_t launch_dense(const GemvParams &p, hipStream_t s) {
-    hipLaunchKernelGGL((k_gemv_dense<HALF, kF32Slices>), dim3((p.rc[0] + kTileRows - 1) / kTileRows),
-                       dim3(kWave * kF32Slices), 0, s, p);
+    const int tiles = (p.rc[0] + kTileRows - 1) / kTileRows;
+    if ((size_t)p.K * (HALF ? 2 : 4) <= kDenseRow)
+        hipLaunchKernelGGL((k_gemv_dense<HALF, 1>), dim3((tiles + kWavesPerWG - 1) / kWavesPerWG), dim3(256), 0, s, p);
+    else
+        hipLaunchKernelGGL((k_gemv_dense<HALF, kF32Slices>), dim3(tiles), dim3(kWave * kF32Slices), 0, s, p);
     return hipGetLastError();
 }
 

@@ -462,7 +462,12 @@ def test_mixed_type_pair_ssm_shapes(m27q, ora, dev, layout):
 @pytest.mark.parametrize("type_name,rc,k,layout", [
     ("Q4_K", 13, 256, 1), ("Q6_K", 7, 768, 0), ("Q8_0", 9, 160, 1), ("Q8_0", 9, 32, 0), ("IQ4_XS", 100, 2304, 1),
     ("Q5_K", 1, 4608, 0), ("Q4_K", 2048, 256, 1), ("Q4_K", 2049, 256, 1), ("Q6_K", 6137, 4096, 1), ("Q6_K", 6145, 4096, 0), ("F16", 1, 8, 0), ("F16", 50, 1000, 0),
-    ("F32", 50, 516, 0), ("F32", 16385, 64, 0)])
+    ("F32", 50, 516, 0), ("F32", 16385, 64, 0)] + [
+    # rows of up to two units or 512 bytes and the next size: a wave per tile and
+    # the split, tiles that the workgroups do not divide
+    ("Q4_K", 2048, 768, 1), ("Q4_K", 2049, 768, 1), ("Q4_K", 100, 512, 1), ("Q4_K", 100, 768, 1),
+    ("Q8_0", 43, 256, 0), ("Q8_0", 43, 288, 0), ("IQ4_XS", 1, 256, 0),
+    ("F16", 4099, 256, 0), ("F16", 4099, 264, 0), ("F32", 4099, 128, 0), ("F32", 4099, 132, 0), ("F32", 65, 4, 0)])
 def test_matvec_f32_split(m27q, ora, dev, type_name, rc, k, layout):
     """Exact-dequantization products with K split over a workgroup's waves:
     fewer units (or 16-byte chunks) than waves, slices of unequal length,
