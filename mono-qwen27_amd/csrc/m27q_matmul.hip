@@ -14,7 +14,7 @@ namespace m27q {
 
 constexpr int kChunkUnits = 4;
 
-template <class T, int LAYOUT, int MT>
+template <class T, int MT>
 __global__ __launch_bounds__(256) void k_matmul_q8(MatmulParams p, int m0) {
     extern __shared__ __align__(16) uint8_t smem[];
     constexpr int CK = kChunkUnits * T::kUnitElems;  // activation values per chunk
@@ -22,7 +22,7 @@ __global__ __launch_bounds__(256) void k_matmul_q8(MatmulParams p, int m0) {
     float *xd = (float *)(smem + MT * CK);           // [MT][CK/32]
     uint32_t *xs = (uint32_t *)(xd + MT * CK / 32);  // [MT][CK/32 * T::kAuxWords]
 
-    using LM = LaneMap<T, LAYOUT>;
+    using LM = LaneMap<T, M27Q_LAYOUT_GGUF>;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = LM::row(lane), c = LM::chunk(lane);
     const int rc = p.rc;
     const int tile = (int)blockIdx.x * kWavesPerWG + wave;
@@ -30,8 +30,7 @@ __global__ __launch_bounds__(256) void k_matmul_q8(MatmulParams p, int m0) {
     const int row = tile * kTileRows + i;
     const int row_ld = row < rc ? row : rc - 1;
     typename T::Lane L(c);
-    const uint8_t *base = LAYOUT == M27Q_LAYOUT_TILED ? p.W + (size_t)tile * p.upr * T::kUnitBytes
-                                                      : p.W + (size_t)row_ld * p.rb * T::kBlockBytes;
+    const uint8_t *base = p.W + (size_t)row_ld * p.rb * T::kBlockBytes;
     float acc[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = 0.f;
@@ -62,10 +61,7 @@ __global__ __launch_bounds__(256) void k_matmul_q8(MatmulParams p, int m0) {
             typename T::Frag f[kChunkUnits];
 #pragma unroll
             for (int k = 0; k < kChunkUnits; ++k)
-                if (u0 + k < p.upr) {
-                    if (LAYOUT == M27Q_LAYOUT_TILED) f[k] = T::load_tiled(base + (size_t)(u0 + k) * T::kUnitBytes, i, c, L);
-                    else f[k] = T::load_gguf(base, u0 + k, p.rb, c, L);
-                }
+                if (u0 + k < p.upr) f[k] = T::load_gguf(base, u0 + k, p.rb, c, L);
 #pragma unroll
             for (int k = 0; k < kChunkUnits; ++k)
                 if (u0 + k < p.upr) {
@@ -87,24 +83,23 @@ __global__ __launch_bounds__(256) void k_matmul_q8(MatmulParams p, int m0) {
     }
 }
 
-template <class T, int LAYOUT, int MT>
+template <class T, int MT>
 static hipError_t launch_mt(const MatmulParams &p, int m0, hipStream_t s) {
     constexpr int CK = kChunkUnits * T::kUnitElems;
     const size_t lds = (size_t)MT * CK + (size_t)MT * CK / 32 * 4 * (1 + T::kAuxWords);
     const int grid = (((p.rc + kTileRows - 1) / kTileRows) + kWavesPerWG - 1) / kWavesPerWG;
-    hipLaunchKernelGGL((k_matmul_q8<T, LAYOUT, MT>), dim3(grid), dim3(256), lds, s, p, m0);
+    hipLaunchKernelGGL((k_matmul_q8<T, MT>), dim3(grid), dim3(256), lds, s, p, m0);
     return hipGetLastError();
 }
 
 template <class T>
 static hipError_t launch_m(const MatmulParams &p, hipStream_t s) {
-    constexpr int L = M27Q_LAYOUT_GGUF;
     for (int m0 = 0; m0 < p.M; m0 += 16) {
         const int left = p.M - m0;
-        const hipError_t e = left <= 2   ? launch_mt<T, L, 2>(p, m0, s)
-                             : left <= 4 ? launch_mt<T, L, 4>(p, m0, s)
-                             : left <= 8 ? launch_mt<T, L, 8>(p, m0, s)
-                                         : launch_mt<T, L, 16>(p, m0, s);
+        const hipError_t e = left <= 2   ? launch_mt<T, 2>(p, m0, s)
+                             : left <= 4 ? launch_mt<T, 4>(p, m0, s)
+                             : left <= 8 ? launch_mt<T, 8>(p, m0, s)
+                                         : launch_mt<T, 16>(p, m0, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
