@@ -81,6 +81,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 
+constexpr int kStepGroups = 4;  // groups of 32 weights per step, half a 256-weight unit
 constexpr int kMinStep = 7;  // powers of two between the parts of a min term's token factor
 constexpr uint32_t kH1024 = 0x64006400u;  // (1024, 1024) in fp16: or-ing an integer below 1024 in adds it
 
@@ -160,13 +161,13 @@ struct WQ4K {
         u4 h;            // d | dmin << 16, scales[12]
         u2 qh;           // Q5_K: qh bytes 8 q ..
     };
-    template <int LAYOUT, int G0, int N>  // groups G0 .. G0 + N - 1 of unit u
+    template <int LAYOUT, int G0>  // groups G0 .. G0 + 3 of unit u
     __device__ static void load(Reg &r, const uint8_t *wp, __amdgpu_buffer_rsrc_t rs, uint32_t base, int i, int q, int u, int) {
         if constexpr (LAYOUT == M27Q_LAYOUT_TILED) {
             const uint32_t s = (uint32_t)u * (uint32_t)kUnitBytes;
 #pragma unroll
-            for (int j = G0 / 2; j < (G0 + N) / 2; ++j) r.q[j] = ld8<0>(rs, base + (uint32_t)(q4k_tqs(i, j) + 8 * q), s);
-            if constexpr (G0 + N == 8) {
+            for (int j = G0 / 2; j < G0 / 2 + 2; ++j) r.q[j] = ld8<0>(rs, base + (uint32_t)(q4k_tqs(i, j) + 8 * q), s);
+            if constexpr (G0 == 4) {
                 r.h = ld16<0>(rs, base + 16u * (uint32_t)i, s);
                 if constexpr (Q5) r.qh = ld8<0>(rs, base + (uint32_t)(kQ5KTQh + 32 * i + 8 * q), s);
             }
@@ -174,8 +175,8 @@ struct WQ4K {
             const uint32_t s = (uint32_t)u * (uint32_t)kBlockBytes;
             constexpr int qs = Q5 ? kQ5KQs : kQ4KHdr;
 #pragma unroll
-            for (int j = G0 / 2; j < (G0 + N) / 2; ++j) r.q[j] = ld8<0>(rs, base + (uint32_t)(qs + 32 * j + 8 * q), s);
-            if constexpr (G0 + N == 8) {
+            for (int j = G0 / 2; j < G0 / 2 + 2; ++j) r.q[j] = ld8<0>(rs, base + (uint32_t)(qs + 32 * j + 8 * q), s);
+            if constexpr (G0 == 4) {
                 r.h = ld16<0>(rs, base, s);
                 if constexpr (Q5) r.qh = ld8<0>(rs, base + (uint32_t)(kQ5KQh + 8 * q), s);
             }
@@ -188,8 +189,8 @@ struct WQ4K {
     // within fp32 wherever the 16-token kernel's, which applies sc later, is:
     // without it rows of magnitude 1e34 to 1e36 came out infinite.
     static constexpr int kDown = 10;
-    template <int G, int LAYOUT>
-    __device__ static AOp<false> operand(const Reg &r, int, uint32_t, const Cst &cst) {
+    template <int G>
+    __device__ static AOp<false> operand(const Reg &r, int, const Cst &cst) {
         constexpr bool odd = G & 1;
         const uint32_t scw = G < 4 ? (r.h.y & 0x3f3f3f3fu) : ((r.h.w & 0x0f0f0f0fu) | ((r.h.y >> 2) & 0x30303030u));
         constexpr uint32_t sel = 0x04000400u | (uint32_t)(G & 3) | ((uint32_t)(G & 3) << 16);
@@ -249,32 +250,25 @@ struct WQ6K {
         u4 sc;
         uint32_t d;
     };
-    template <int LAYOUT, int G0, int N>
+    template <int LAYOUT, int G0>
     __device__ static void load(Reg &r, const uint8_t *wp, __amdgpu_buffer_rsrc_t rs, uint32_t base, int i, int q, int u, int) {
-        // ql chunks 2 h, 2 h + 1 serve all four groups of half h: (re)loaded with its last ones
-        constexpr int h0 = G0 / 4, h1 = (G0 + N) / 4;
+        constexpr int h = G0 / 4;  // half of the unit
         if constexpr (LAYOUT == M27Q_LAYOUT_TILED) {
             const uint32_t s = (uint32_t)u * (uint32_t)kUnitBytes;
 #pragma unroll
-            for (int h = h0; h < h1; ++h) {
-#pragma unroll
-                for (int x = 0; x < 2; ++x)
-                    r.ql[2 * h + x] = ld8<0>(rs, base + (uint32_t)(kQ6KTQl + 128 * i + 64 * h + 32 * x + 8 * q), s);
-                r.qh[h] = ld8<0>(rs, base + (uint32_t)(kQ6KTQh + 64 * i + 32 * h + 8 * q), s);
-            }
-            if constexpr (G0 + N == 8) {
+            for (int x = 0; x < 2; ++x)
+                r.ql[2 * h + x] = ld8<0>(rs, base + (uint32_t)(kQ6KTQl + 128 * i + 64 * h + 32 * x + 8 * q), s);
+            r.qh[h] = ld8<0>(rs, base + (uint32_t)(kQ6KTQh + 64 * i + 32 * h + 8 * q), s);
+            if constexpr (G0 == 4) {
                 r.sc = ld16<0>(rs, base + (uint32_t)(kQ6KTSc + 16 * i), s);
                 r.d = bld_u16<0>(rs, base + (uint32_t)(kQ6KTD + 2 * i), s);
             }
         } else {
             const uint8_t *blk = wp + (base + (uint32_t)u * (uint32_t)kBlockBytes);
 #pragma unroll
-            for (int h = h0; h < h1; ++h) {
-#pragma unroll
-                for (int x = 0; x < 2; ++x) r.ql[2 * h + x] = ldu8(blk + kQ6KQl + 64 * h + 32 * x + 8 * q);
-                r.qh[h] = ldu8(blk + kQ6KQh + 32 * h + 8 * q);
-            }
-            if constexpr (G0 + N == 8) {
+            for (int x = 0; x < 2; ++x) r.ql[2 * h + x] = ldu8(blk + kQ6KQl + 64 * h + 32 * x + 8 * q);
+            r.qh[h] = ldu8(blk + kQ6KQh + 32 * h + 8 * q);
+            if constexpr (G0 == 4) {
                 r.sc = ldu16(blk + kQ6KSc);
                 r.d = *(const uint16_t *)(blk + kQ6KD);
             }
@@ -282,8 +276,8 @@ struct WQ6K {
     }
     // sc (q - 32) of group G as two fp16 operands: their product rounded to
     // fp16, and the remainder (an FMA; exact).
-    template <int G, int LAYOUT>
-    __device__ static AOp<true> operand(const Reg &r, int q, uint32_t off, const Cst &cst) {
+    template <int G>
+    __device__ static AOp<true> operand(const Reg &r, int q, const Cst &cst) {
         constexpr int h = G / 4, rr = G % 4;
         constexpr bool hi = rr >= 2;
         const u2 ql = r.ql[2 * h + (rr & 1)], qh = r.qh[h];
@@ -323,28 +317,28 @@ struct WQ80 {
     static constexpr int kUnitBytes = kQ80Unit, kBlockBytes = kQ80Bytes;
     struct Reg {
         u2 q[8];
-        uint32_t d[8];  // TILED: words 0, 1 / 4, 5 hold two scales each; GGUF: one each
+        uint32_t d[8];  // TILED: words 0, 2, 4, 6 hold two scales each; GGUF: one each
     };
-    template <int LAYOUT, int G0, int N>
+    template <int LAYOUT, int G0>
     __device__ static void load(Reg &r, const uint8_t *wp, __amdgpu_buffer_rsrc_t rs, uint32_t base, int i, int q, int u, int rb) {
         if constexpr (LAYOUT == M27Q_LAYOUT_TILED) {
             const int nu = (rb + kQ80UnitBlocks - 1) / kQ80UnitBlocks;
             const uint32_t s = (uint32_t)min(2 * u + G0 / 4, nu - 1) * (uint32_t)kUnitBytes;
 #pragma unroll
-            for (int g = G0; g < G0 + N; ++g) r.q[g] = ld8<0>(rs, base + (uint32_t)(128 * i + 32 * (g & 3) + 8 * q), s);
-            r.d[G0 / 2 * 2] = bld_u32<0>(rs, base + (uint32_t)(kQ80TD + 8 * i + 2 * (G0 & 3)), s);
-            if constexpr (N == 4) r.d[G0 / 2 * 2 + 2] = bld_u32<0>(rs, base + (uint32_t)(kQ80TD + 8 * i + 4), s);
+            for (int g = G0; g < G0 + 4; ++g) r.q[g] = ld8<0>(rs, base + (uint32_t)(128 * i + 32 * (g & 3) + 8 * q), s);
+            r.d[G0] = bld_u32<0>(rs, base + (uint32_t)(kQ80TD + 8 * i), s);
+            r.d[G0 + 2] = bld_u32<0>(rs, base + (uint32_t)(kQ80TD + 8 * i + 4), s);
         } else {
 #pragma unroll
-            for (int g = G0; g < G0 + N; ++g) {
+            for (int g = G0; g < G0 + 4; ++g) {
                 const uint8_t *blk = wp + (base + (uint32_t)min(8 * u + g, rb - 1) * (uint32_t)kBlockBytes);
                 r.q[g] = ldu8(blk + 2 + 8 * q);
                 r.d[g] = *(const uint16_t *)blk;
             }
         }
     }
-    template <int G, int LAYOUT>
-    __device__ static long operand(const Reg &r, int, uint32_t, int, int) {
+    template <int G>
+    __device__ static long operand(const Reg &r) {
         return __builtin_bit_cast(long, r.q[G]);
     }
     // Group G's scale of row c (0 past the row's blocks).
@@ -364,17 +358,17 @@ struct WIQ4XS {
         uint32_t q[8];  // qs bytes 4 q .. + 4 of each group
         u2 hd;          // d | scales_h << 16, scales_l[4]
     };
-    template <int LAYOUT, int G0, int N>
+    template <int LAYOUT, int G0>
     __device__ static void load(Reg &r, const uint8_t *wp, __amdgpu_buffer_rsrc_t rs, uint32_t base, int i, int q, int u, int) {
         constexpr bool kT = LAYOUT == M27Q_LAYOUT_TILED;
         const uint32_t s = (uint32_t)u * (uint32_t)(kT ? kUnitBytes : kBlockBytes);
         const uint32_t qs = base + (uint32_t)(kT ? 128 * i : kIQ4XSQs) + 4u * (uint32_t)q;
 #pragma unroll
-        for (int g = G0; g < G0 + N; ++g) r.q[g] = bld_u32<0>(rs, qs + 16u * (uint32_t)g, s);
-        if constexpr (G0 + N == 8) r.hd = ld8<0>(rs, base + (uint32_t)(kT ? kIQ4XSTHdr + 8 * i : 0), s);
+        for (int g = G0; g < G0 + 4; ++g) r.q[g] = bld_u32<0>(rs, qs + 16u * (uint32_t)g, s);
+        if constexpr (G0 == 4) r.hd = ld8<0>(rs, base + (uint32_t)(kT ? kIQ4XSTHdr + 8 * i : 0), s);
     }
-    template <int G, int LAYOUT>
-    __device__ static long operand(const Reg &r, int, uint32_t, int, int) {
+    template <int G>
+    __device__ static long operand(const Reg &r) {
         const uint32_t w = r.q[G];
         return __builtin_bit_cast(long, u2{iq4_lut(w & 0x0f0f0f0fu), iq4_lut((w >> 4) & 0x0f0f0f0fu)});
     }
@@ -389,16 +383,15 @@ struct WIQ4XS {
 
 constexpr uint32_t kPast = 0xffffff00u;  // past every activation buffer (below 2^27 bytes)
 
-// Launch shapes: RW row waves x KW slices of K, at most RSM sets per wave, GS
-// groups per step.
-template <int RW_, int KW_, int RSM_, int GS_>
+// Launch shapes: RW row waves x KW slices of K, at most RSM sets per wave.
+template <int RW_, int KW_, int RSM_>
 struct Shape {
-    static constexpr int RW = RW_, KW = KW_, RSM = RSM_, GS = GS_, W = RW_ * KW_;
+    static constexpr int RW = RW_, KW = KW_, RSM = RSM_, W = RW_ * KW_;
 };
 
 template <class T, int NT, class SH>
 struct Wide {
-    static constexpr int RW = SH::RW, KW = SH::KW, RSM = SH::RSM, GS = SH::GS, W = SH::W;
+    static constexpr int RW = SH::RW, KW = SH::KW, RSM = SH::RSM, GS = kStepGroups, W = SH::W;
     static constexpr int NB = RW == 1 ? 1 : 2;   // step buffers
     // activation loads in flight, in steps: a step of one set is shorter than
     // their latency
@@ -649,8 +642,7 @@ __global__ __launch_bounds__(kWave *SH::W, SH::W / 4) void k_matmul_wide(MatmulM
                 for (int t = 0; t < NT; ++t) b[t] = *(const h8 *)(xc + (GI * NT + t) * (kWave * 16) + xo[GI]);
 #pragma unroll
                 for (int s = 0; s < NS; ++s) {
-                        const uint32_t off = kT ? 0u : base[s] + (uint32_t)u * (uint32_t)T::kBlockBytes;
-                        const auto a = T::template operand<G, LAYOUT>(w[s], q, off, cst);
+                        const auto a = T::template operand<G>(w[s], q, cst);
                         f4 d[NT];
 #pragma unroll
                         for (int t = 0; t < NT; ++t)
@@ -675,7 +667,7 @@ __global__ __launch_bounds__(kWave *SH::W, SH::W / 4) void k_matmul_wide(MatmulM
                 for (int t = 0; t < NT; ++t) b[t] = __builtin_bit_cast(long, *(const u2 *)(xc + (GI * NT + t) * (kWave * 8) + xo[GI]));
 #pragma unroll
                 for (int s = 0; s < NS; ++s) {
-                        const long a = T::template operand<G, LAYOUT>(w[s], q, base[s], u, p.rb);
+                        const long a = T::template operand<G>(w[s]);
                         const float f = T::template factor<G, LAYOUT>(w[s], u, p.rb);
                         i4 d[NT];
 #pragma unroll
@@ -744,7 +736,7 @@ __global__ __launch_bounds__(kWave *SH::W, SH::W / 4) void k_matmul_wide(MatmulM
     auto reload = [&](auto st, int u) __attribute__((always_inline)) {
 #pragma unroll
         for (int s = 0; s < NS; ++s)
-            T::template load<LAYOUT, decltype(st)::value * GS, GS>(w[s], wp[s], rs[s], base[s], ri[s], q, min(u + 1, ub - 1), p.rb);
+            T::template load<LAYOUT, decltype(st)::value * GS>(w[s], wp[s], rs[s], base[s], ri[s], q, min(u + 1, ub - 1), p.rb);
     };
 
     if (ua < ub) {
@@ -753,7 +745,7 @@ __global__ __launch_bounds__(kWave *SH::W, SH::W / 4) void k_matmul_wide(MatmulM
 #pragma unroll
         for (int s = 0; s < NS; ++s)
             unroll<NST>([&](auto st) __attribute__((always_inline)) {
-                    T::template load<LAYOUT, decltype(st)::value * GS, GS>(w[s], wp[s], rs[s], base[s], ri[s], q, ua, p.rb);
+                    T::template load<LAYOUT, decltype(st)::value * GS>(w[s], wp[s], rs[s], base[s], ri[s], q, ua, p.rb);
                 });
         commit(0, Int<0>{}, 0);
         issue(ua * NST + C::DP, Int<C::DP>{});
@@ -845,10 +837,10 @@ hipError_t launch_wide_t(const MatmulMultiParams &p, int grid, hipStream_t s) {
     return hipGetLastError();
 }
 
-using ShapeFew = Shape<1, 8, 1, 4>;
-using ShapePair = Shape<2, 4, 1, 4>;
-using ShapeMid = Shape<2, 4, 3, 4>;
-using ShapeMany = Shape<4, 2, 3, 4>;
+using ShapeFew = Shape<1, 8, 1>;
+using ShapePair = Shape<2, 4, 1>;
+using ShapeMid = Shape<2, 4, 3>;
+using ShapeMany = Shape<4, 2, 3>;
 
 // Grid and split by the number S of 16-row sets per CU.
 template <class T, int NT, int LAYOUT>
