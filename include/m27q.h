@@ -254,20 +254,25 @@ M27Q_API m27q_status m27q_matvec_f32(const m27q_weight *w, const float *x, float
 /* Y[m][r] = sum_k W[r][k] * xq[m][k] (+ residual[m][r]) for m < M, 1 <= M <= 64,
  * xq from m27q_quant_act with this M (the whole buffer of m27q_act_bytes(M,
  * K) bytes: Q8_0 weights whose K is not a multiple of 128 read up to 96 bytes
- * past the last row's codes); Y is [M][row_count].  M = 2 runs on the GEMV
- * structure, from M = 3 TILED weights and GGUF-layout Q4_K / Q5_K / Q6_K
- * weights on int8 MFMA (v_mfma_i32_16x16x32_i8, up to 16 activation rows per
- * launch), other GGUF-layout weights on a packed-int8-dot path; M = 1 is
- * m27q_matvec_q8.  No reference
- * counterpart: the reference runs prefill and decode one token at a time
- * (src/mono27b_chat.cpp:399-403); results equal M independent M = 1 products
- * up to fp32 rounding. */
+ * past the last row's codes); Y is [M][row_count].  M = 1 is m27q_matvec_q8.
+ * M = 2 runs on the GEMV structure, TILED Q4_K / Q5_K excepted; up to 16 rows,
+ * those and, from M = 3, TILED weights and GGUF-layout Q4_K / Q5_K / Q6_K run on
+ * int8 MFMA (v_mfma_i32_16x16x32_i8), GGUF-layout Q8_0 / IQ4_XS on a
+ * packed-int8-dot path.  From 17 rows (GGUF-layout Q8_0 / IQ4_XS from 5) one
+ * launch takes all rows in one pass over the weights (fp16 and bf16 MFMA with
+ * exact integer operands, int8 MFMA for Q8_0 / IQ4_XS) where that is faster, by
+ * type, layout, rows and K, and always past 32; otherwise there is a launch per
+ * 16 rows of the former kind.  No reference counterpart: the reference runs
+ * prefill and decode one token at a time (src/mono27b_chat.cpp:399-403); results
+ * equal M independent M = 1 products up to fp32 rounding. */
 M27Q_API m27q_status m27q_matmul_q8(const m27q_weight *w, int M, const void *xq, float *Y,
                                     const float *residual, hipStream_t stream);
 
 /* Up to 4 weights of one K on the same M activation rows: Ys[i] = X W[i]^T
- * ([M][row_count_i] each), one launch per (type, layout) group as in
- * m27q_matvec_q8_multi (GGUF-layout Q8_0 / IQ4_XS: one launch per weight).
+ * ([M][row_count_i] each), launched per (type, layout) group as in
+ * m27q_matvec_q8_multi (GGUF-layout Q8_0 / IQ4_XS on the packed-int8-dot path:
+ * per weight).  How K is split, and so the rounding, follows the group's total
+ * rows: a weight's result need not equal the single call's bit for bit.
  * The small-M counterpart of m27q_matvec_q8_multi (q/k/v, gate/up of a
  * verify batch). */
 M27Q_API m27q_status m27q_matmul_q8_multi(int n, const m27q_weight *ws, int M, const void *xq, float *const *Ys,
@@ -320,7 +325,8 @@ M27Q_API m27q_status m27q_topk_noalloc(const float *logits, int n, int k, int32_
 
 /* On-device token choice from m27q_topk's candidates (idx/val in rank order,
  * 1 <= k <= 64), the steps of sample() (src/mono27b_chat.cpp:203-270) after its
- * top-k: temperature <= 0 gives idx[0] (the argmax, first index on ties);
+ * top-k: temperature <= 0 gives idx[0] (the argmax, first index on ties; nothing
+ * else is read then);
  * otherwise p_i = e^((val_i - val_0) / temperature) (the fixed exp of
  * m27q_quant_act_gated; 0 below e^-87), normalized; candidates
  * with p_i < p_0 * min_p are dropped; top_p < 1 keeps the shortest prefix whose

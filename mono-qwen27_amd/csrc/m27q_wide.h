@@ -37,21 +37,32 @@
 // Work.  8 waves, one workgroup per CU: RW row waves x KW slices of K.  A
 // workgroup owns a run of 16-row sets (spread evenly over the grid), dealt to
 // its row waves, at most RSM each.  The row waves of a K slice share its
-// activations, converted and laid out in operand order in LDS GS groups at a
-// time (double-buffered, one barrier per step; a slice of one wave needs
-// neither), while each wave's weights stream from memory straight into
-// registers, one 256-weight unit ahead.  The KW partial sums are added in LDS in
-// slice order.
+// activations, converted and laid out in operand order in LDS four groups at a
+// time (a step; double-buffered, one barrier per step; a slice of one wave has
+// one buffer and no barrier), while each wave's weights stream from memory
+// straight into registers, asked for one 256-weight unit ahead.  The KW partial
+// sums are added in LDS in slice order.
+//
+// What holds it back now, by the compiler's output (VGPRs, spills, instructions
+// and waits of the loops):
+//   - a step is conditional (slices differ by a unit), so the wait counts merge
+//     over both paths and each step drains every load in flight (vmcnt(0)) before
+//     its last groups: the weights are not a whole unit ahead in effect.  The next
+//     unit's scales, needed by its first group, are asked for last;
+//   - Q6_K with four token tiles and three sets per wave (M = 49 to 64 past two
+//     sets per CU) does not fit 256 registers and spills 14 to 51 of them: 17408 x
+//     5120 42.7 us at M = 48, 84.6 at M = 64 (107.1 in launches of 16 tokens).
 //
 // What was measured on the way (gate/up, 2 x 17408 x 5120 Q4_K, and down, 5120
-// x 17408 Q6_K with the residual, at M = 64; kernel trace):
-//   - launches of 16 tokens of the MFMA kernel: 130 and 114 us (four each);
-//     this kernel 62 and 66;
+// x 17408 Q6_K, at M = 64; replays of a graph; what was slower, on the loop as it
+// is, so an unconditional one may decide otherwise):
+//   - four launches of 16 tokens of the MFMA kernel: 115 and 103 us; this kernel
+//     59 and 65;
 //   - the vector and matrix instructions of a wave pair add up (they hardly
-//     overlap): down's 511 vector instructions and 64 MFMAs per unit and set
-//     are about 47 of its 66 us.  Dealing MFMAs between vector instructions of
-//     other groups (schedule groups, software pipelining over sets) was slower:
-//     75 against 67 us on gate/up;
+//     overlap): down's 543 vector instructions of 4 cycles and 64 MFMAs of 16 per
+//     unit (and set, of one per wave) are about 47 of its 65 us.  Dealing MFMAs
+//     between vector instructions of other groups (schedule groups, software
+//     pipelining over sets) was slower: 75 against 67 us on gate/up (traced);
 //   - loads must touch few 128-byte lines: a step of 4 groups reads each
 //     token's 128 codes as one line (2 groups, half a line: Q4_K 5120 x 17408
 //     87 us against 58), and the weights' 8-byte pieces of a line come in

@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 from gpu_util import act_host, int_dot_tol, say, to_dev, to_host
+from test_oracle import random_blocks
 
 pytestmark = pytest.mark.gpu
 
@@ -26,12 +27,12 @@ CASES = [  # type, rows, K, M, layout
     ("IQ4_XS", 40, 512, 3, 0),
     # MFMA with two 16-row sets per tile (M <= 8 and >= 128 sets of 32 rows):
     # a partial last set (8200 rows), a partial Q8_0 unit (K = 160), every
-    # type, and 24 tokens (one 16-token launch, then one packed 8-token launch)
+    # type; 24 tokens on the wide kernel
     ("Q4_K", 8200, 512, 5, 1), ("Q4_K", 8192, 512, 8, 1), ("Q4_K", 8192, 512, 24, 1),
     ("Q6_K", 8200, 768, 7, 1), ("Q8_0", 8200, 160, 6, 1), ("Q5_K", 8192, 512, 8, 1),
     ("IQ4_XS", 8200, 512, 6, 1),
     # gate-sized rows at M = 3 (two sets per tile), the down shape at M = 12
-    # (padding tokens in a 16-token launch), 17 tokens (16, then 1 on two sets)
+    # (padding tokens in a 16-token launch), 17 tokens on the wide kernel
     ("Q4_K", 17408, 5120, 3, 1), ("Q6_K", 5120, 17408, 12, 1), ("Q4_K", 8192, 512, 17, 1),
     # few tokens with balanced tiling on 256 CUs (rows under 40 units) on the
     # GEMV-structured kernel (Q6_K), and the same shapes on MFMA with direct
@@ -42,8 +43,7 @@ CASES = [  # type, rows, K, M, layout
     ("Q4_K", 13, 256, 2, 1), ("Q5_K", 8200, 512, 2, 1), ("Q4_K", 17408, 1024, 2, 1),
     # resident activation rows (16-token launches with >= 4 row sets per CU:
     # 1025 sets of 16 rows on 256 CUs), every type, a partial last set, a
-    # partial Q8_0 unit (K = 1056), and 16 + 9 tokens (the resident launch,
-    # then the per-unit staging one)
+    # partial Q8_0 unit (K = 1056); 25 and 32 tokens on the wide kernel
     ("Q4_K", 16390, 1024, 16, 1), ("Q6_K", 16390, 1024, 16, 1), ("Q8_0", 16390, 1056, 16, 1),
     ("Q5_K", 16390, 1024, 25, 1), ("IQ4_XS", 16390, 1024, 32, 1),
     # two row sets per tile over 1025 sets of 32 rows (a last set of 8 rows),
@@ -52,7 +52,8 @@ CASES = [  # type, rows, K, M, layout
     ("Q5_K", 32776, 512, 3, 1), ("IQ4_XS", 32776, 512, 8, 1),
     # GGUF-layout K-quants on the MFMA kernel, staged from the row blocks:
     # from M = 2, two-set tiles with a partial last set, 16-token resident
-    # launches (Q6_K: the per-unit kernel) and padding tokens; Q6_K rows of an
+    # launches (Q6_K: the per-unit kernel), 16 + 3 tokens (257 sets) and padding
+    # tokens, 25 tokens on the wide kernel; Q6_K rows of an
     # odd block count (K = 768, 2304: every other row starts 2 bytes past a
     # multiple of 4) and the down shape
     ("Q4_K", 6144, 5120, 2, 0), ("Q4_K", 8200, 512, 6, 0), ("Q4_K", 16390, 1024, 16, 0), ("Q4_K", 4100, 1024, 19, 0),
@@ -92,7 +93,8 @@ def test_matmul_vs_oracle(m27q, ora, dev, type_name, rc, k, M, layout):
 @pytest.mark.parametrize("M", [2, 5, 16, 19])
 def test_matmul_multi_vs_oracle(m27q, ora, dev, M):
     """q/k/v-shaped weights on one activation in one launch, each against the
-    integer-dot oracle (row subsets), across the 16-token launch boundary."""
+    integer-dot oracle (row subsets), across the 16-token launch boundary (M = 19:
+    a launch of 16 tokens and one of 3)."""
     import torch
     k, shapes = 5120, [6144, 1024, 1024]
     wbs = [ora.synth_weights(m27q.Q4_K, rc, k, seed=60 + i) for i, rc in enumerate(shapes)]
@@ -113,10 +115,10 @@ def test_matmul_multi_vs_oracle(m27q, ora, dev, M):
 
 @pytest.mark.parametrize("M,rows", [(16, 8200), (32, 8200), (7, 16400)])
 def test_matmul_multi_resident_vs_oracle(m27q, ora, dev, M, rows):
-    """Two weights of one K in one launch over 1026 row sets: at M = 16 and 32
-    the resident-activation kernel (the second matrix's sets following the
-    first's in the workgroups' runs), at M = 7 the two-set per-unit kernel;
-    each against the integer-dot oracle."""
+    """Two weights of one K in one launch over 1026 row sets: at M = 16 the
+    resident-activation kernel (the second matrix's sets following the first's
+    in the workgroups' runs), at M = 32 the wide kernel, at M = 7 the two-set
+    per-unit kernel; each against the integer-dot oracle."""
     import torch
     k, shapes = 1024, [rows, rows]
     wbs = [ora.synth_weights(m27q.Q4_K, rc, k, seed=70 + i) for i, rc in enumerate(shapes)]
@@ -139,8 +141,8 @@ def test_matmul_multi_resident_vs_oracle(m27q, ora, dev, M, rows):
 def test_matmul_multi_gguf_vs_oracle(m27q, ora, dev, M):
     """GGUF-layout weights through the multi entry point: Q4_K q/k/v-shaped
     weights in one MFMA launch, then a mixed group (Q6_K on the MFMA kernel,
-    Q8_0 on the per-weight VALU kernel) on the same activation; every token
-    row of each output against the integer-dot oracle."""
+    Q8_0 on the wide one; M = 2 on the few-token kernel) on the same activation;
+    every token row of each output against the integer-dot oracle."""
     import torch
     k = 1536
     spec = [("Q4_K", 6144, 80), ("Q4_K", 1024, 81), ("Q4_K", 1024, 82)]
@@ -176,7 +178,7 @@ def test_gguf_two_byte_aligned_base(m27q, ora, dev, type_name, rc, k):
     products (quantized and fp32 x; one- and two-tile waves read Q6_K's fields
     as shifted dwords or halfwords) and the small-M products (Q6_K: the MFMA
     kernel with one- and two-set tiles, whose staging reads dwords from the
-    4-aligned address below each chunk; Q8_0: the VALU kernel), every token
+    4-aligned address below each chunk; Q8_0: the wide kernel), every token
     row against the integer-dot oracle."""
     import torch
     t = getattr(m27q, type_name)
@@ -213,7 +215,8 @@ WIDE = [  # type, rows, K, M, layout: the wide kernel's launch shapes on 256 CUs
     # (seven waves without work), a unit count the slices do not divide
     ("Q4_K", 13, 256, 17, 1), ("Q5_K", 40, 2304, 33, 0), ("Q6_K", 40, 2304, 64, 1), ("Q6_K", 13, 256, 49, 0),
     ("IQ4_XS", 40, 512, 64, 1), ("Q8_0", 13, 32, 17, 1), ("Q8_0", 40, 1056, 64, 1), ("Q8_0", 13, 160, 9, 0),
-    ("Q8_0", 13, 32, 5, 0), ("IQ4_XS", 13, 256, 5, 0),
+    # ... of 5 and 8 rows
+    ("Q8_0", 13, 384, 5, 0), ("IQ4_XS", 13, 1280, 5, 0), ("Q8_0", 4095, 416, 8, 0),
     # two row waves of at most one set: an odd set count (257: a wave without a
     # set), a partial last 8-row tile and set
     ("Q4_K", 4100, 1024, 33, 1), ("Q4_K", 4100, 256, 64, 0), ("Q5_K", 4100, 512, 48, 1), ("Q6_K", 4100, 768, 64, 0),
@@ -224,13 +227,32 @@ WIDE = [  # type, rows, K, M, layout: the wide kernel's launch shapes on 256 CUs
     # four row waves of up to three sets: just above 6 sets per CU, two rounds
     ("Q4_K", 24600, 512, 64, 1), ("Q5_K", 50001, 256, 33, 1), ("Q6_K", 24600, 256, 33, 0), ("Q8_0", 24600, 160, 64, 1),
     ("IQ4_XS", 24600, 256, 20, 0), ("Q4_K", 24600, 256, 17, 0),
+    # 9 and 16 rows on two row waves of up to three sets (521 and 770 sets) and on
+    # four (1538), partial last sets
+    ("Q8_0", 8330, 416, 9, 0), ("Q8_0", 12310, 1024, 16, 0), ("Q8_0", 24605, 2560, 9, 0),
+    ("IQ4_XS", 8330, 512, 16, 0), ("IQ4_XS", 12310, 1280, 9, 0), ("IQ4_XS", 24605, 1280, 16, 0),
+]
+# 5 rows of a short K, which the VALU kernel keeps
+VALU_SHORT = [("Q8_0", 13, 32, 5, 0), ("IQ4_XS", 13, 256, 5, 0)]
+# 17 to 32 rows on the MFMA kernel (257 and 385 sets; a launch of 16 rows, then one
+# of up to 8 rows on two-set tiles or of more on one-set ones), partial last sets;
+# 3075 sets, past 12 per CU: the resident kernel, then one row
+TWO_LAUNCHES = [
+    ("Q4_K", 4100, 1024, 17, 1), ("Q4_K", 4100, 1024, 24, 1), ("Q4_K", 4100, 1024, 32, 1),
+    ("Q5_K", 4100, 512, 17, 1), ("Q5_K", 4100, 512, 24, 1), ("Q5_K", 4100, 512, 32, 1), ("Q5_K", 4100, 512, 24, 0),
+    ("Q6_K", 4100, 768, 17, 1), ("Q6_K", 4100, 768, 24, 1), ("Q6_K", 4100, 768, 32, 1),
+    ("Q6_K", 4100, 768, 17, 0), ("Q6_K", 6150, 768, 32, 0), ("Q4_K", 4100, 512, 32, 0),
+    ("Q8_0", 4100, 1056, 17, 1), ("Q8_0", 4100, 1056, 24, 1), ("Q8_0", 4100, 1056, 32, 1),
+    ("IQ4_XS", 4100, 512, 17, 1), ("IQ4_XS", 6150, 512, 24, 1), ("IQ4_XS", 6150, 512, 32, 1),
+    ("Q8_0", 49195, 544, 17, 1),
 ]
 
 
-@pytest.mark.parametrize("type_name,rc,k,M,layout", WIDE)
+@pytest.mark.parametrize("type_name,rc,k,M,layout", WIDE + VALU_SHORT + TWO_LAUNCHES)
 def test_wide_vs_oracle(m27q, ora, dev, type_name, rc, k, M, layout):
-    """One launch of up to 64 rows (its first, last and tile-edge tokens, with a
-    residual) against the integer-dot oracle.  The scaled integer sums are
+    """One launch of up to 64 rows, or the launches of 16 that it replaces
+    elsewhere (the first, last and tile-edge tokens, with a residual) against
+    the integer-dot oracle.  The scaled integer sums are
     exact, so what differs is the order of the fp32 sums over groups and
     blocks: the bar of every product (int_dot_tol)."""
     import torch
@@ -372,3 +394,64 @@ def test_gguf_valu_16_rows(m27q, ora, dev, type_name, rc, k, M):
     for m in range(M):
         want, nrm = ora.gemv_act(t, wb, rb, rc, q[m], d[m], s[m])
         assert (np.abs(got[m] - res[m] - want) <= int_dot_tol(nrm) + 1e-6 * np.abs(res[m])).all(), m
+
+
+def test_resident_second_launch(m27q, ora, dev):
+    """32 rows in two launches of the resident-activation kernel: IQ4_XS, more
+    than 12 sets per CU and a long K (random bytes: 194 MB of weights)."""
+    import torch
+    rc, k, M = 49200, 7424, 32
+    rb = k // 256
+    wb = random_blocks(ora, ora.IQ4_XS, rb * rc, np.random.default_rng(12))
+    w = m27q.Weight.upload(wb.reshape(-1), m27q.IQ4_XS, rb, rc, m27q.TILED, dev)
+    act = m27q.Act(M, k, dev)
+    m27q.quant_act(to_dev(np.random.default_rng(13).standard_normal((M, k)).astype(np.float32), dev), act)
+    Y = torch.empty((M, rc), dtype=torch.float32, device=dev)
+    say("resident twice", rc, k, M)
+    m27q.matmul_q8(w, act, Y)
+    got = to_host(Y).astype(np.float64)
+    q, d, s = act_host(m27q, act)
+    for m in (0, 15, 16, 31):
+        want, nrm = ora.gemv_act(ora.IQ4_XS, wb, rb, rc, q[m], d[m], s[m])
+        assert (np.abs(got[m] - want) <= int_dot_tol(nrm)).all(), m
+
+
+@pytest.mark.parametrize("type_name,layout", [(t, lay) for t in ("Q4_K", "Q5_K", "Q6_K", "Q8_0", "IQ4_XS") for lay in (0, 1)])
+@pytest.mark.parametrize("rc,M", [(100, 17), (4100, 33), (8210, 64), (24600, 40)])
+def test_wide_exact_integers(m27q, ora, dev, type_name, layout, rc, M):
+    """Weights of block scale 1 (scales, mins and codes at their extremes among
+    random ones) times codes with one power-of-two scale: every product and sum
+    is a multiple of it below 2^24, so the results are exact, on each launch
+    shape.  A lost bit of an operand (Q6_K's second fp16 value, a min term's
+    third part) shows."""
+    import torch
+    t, k = getattr(m27q, type_name), 512
+    rb = k // m27q.BLOCK_ELEMS[t]
+    rng = np.random.default_rng(rc + M)
+    b = rng.integers(0, 256, size=(rc * rb, ora.TYPE_SIZE[t]), dtype=np.uint8)
+    one = np.frombuffer(np.float16(1).tobytes(), np.uint8)
+    b[rng.random(b.shape) < 0.2] = 0x80 if type_name == "Q6_K" else 0xff  # Q6_K: scale -128 ...
+    b[rng.random(b.shape) < 0.2] = 0x00                                   # ... and code -32
+    off = 208 if type_name == "Q6_K" else 0
+    b[:, off:off + 2] = one
+    if type_name in ("Q4_K", "Q5_K"):
+        b[:, 2:4] = one
+    wb = b.reshape(rc, -1)
+    w = m27q.Weight.upload(wb.reshape(-1), t, rb, rc, layout, dev)
+    # two codes per group, one of them +-127 (so that the group's scale is 2^-3);
+    # 16 groups x 2 x 127 x 4096 = 16,646,144 < 2^24
+    X = np.zeros((M, k), np.float32)
+    for m in range(M):
+        for g in range(0, k, 32):
+            i, j = rng.choice(32, 2, replace=False)
+            X[m, g + i], X[m, g + j] = rng.choice([-127, 127]), rng.integers(-127, 128)
+    act = m27q.Act(M, k, dev)
+    m27q.quant_act(to_dev(X / 8, dev), act)
+    q, d, s = act_host(m27q, act)
+    assert np.array_equal(q, X) and (d == 0.125).all()
+    Y = torch.empty((M, rc), dtype=torch.float32, device=dev)
+    say("wide exact", type_name, layout, rc, M)
+    m27q.matmul_q8(w, act, Y)
+    # whole numbers up to 2^24: exact in a float64 product
+    want = X.astype(np.float64) @ ora.dequant(t, wb, rb, rc).astype(np.float64).T / 8
+    assert np.array_equal(to_host(Y).astype(np.float64), want)

@@ -3,10 +3,11 @@ integer-dot oracle: random type, layout, row count (ragged tiles), K (whole
 blocks, ragged Q8_0 units), token count M up to the entry points' 64 (the few-token GEMV, both MFMA
 packings, 16-token launches and their remainders), fp32 or quantized
 activations, residual, multi-weight launches of mixed types and the SwiGLU
-epilogue.  Those draw at most 3000 rows, too few for the resident-activation
-kernel (16-token launches over >= 4 row sets of 16 per CU: 16369 rows on 256
-CUs); a third set of seeds draws 16400-20000 rows and 16-40 tokens for it,
-every token row checked.  The fixed cases elsewhere pin the
+epilogue.  Those draw at most 3000 rows (at most one row set of 16 per CU, so
+past 16 tokens the wide kernel's one-wave slices); a third set of seeds draws
+16400-20000 rows (more than 4 row sets per CU on 256 CUs) and 16-40 tokens:
+the resident-activation kernel at 16, the wide kernel's two and four row waves
+past them, every token row checked.  The fixed cases elsewhere pin the
 benched shapes and the edges the kernels were written for; these cover the
 combinations between them (any layout, except multi-weight launches of
 several tokens, which take TILED weights).  A second set of seeds draws the
@@ -58,9 +59,8 @@ def test_random_bytes_vs_oracle(m27q, ora, dev, seed):
 @pytest.mark.parametrize("seed", range(9000, 9006))
 def test_random_resident_vs_oracle(m27q, ora, dev, seed):
     """Random type and layout, 16400-20000 rows (ragged last set), small K,
-    16-40 tokens (resident 16-token launches, then the remainder on the
-    per-unit kernel; GGUF-layout Q8_0 / IQ4_XS on the VALU kernel), one or
-    two weights of one K; every token row against the oracle."""
+    16-40 tokens (16: the resident kernel; more: the wide one), one or two
+    weights of one K; every token row against the oracle."""
     import torch
     r = np.random.default_rng(3000 + seed)
     t = TYPES[r.integers(len(TYPES))]

@@ -66,6 +66,16 @@ def wins(tmp_path_factory):
     return run
 
 
+def test_gpu_cases_take_the_kernel_they_name(wins):
+    """The parity tests' lists: the wide kernel's cases reach it, the others don't."""
+    import test_gpu_matmul as g
+    order = lambda cases: [(t, layout, rows, K, M) for t, rows, K, M, layout in cases]  # noqa: E731
+    assert [c for c, w in zip(g.WIDE, wins(order(g.WIDE))) if not w] == []
+    other = g.VALU_SHORT + g.TWO_LAUNCHES
+    assert [c for c, w in zip(other, wins(order(other))) if w] == []
+    assert wins([("IQ4_XS", 1, 49200, 7424, 32)]) == [False]
+
+
 def test_products_measured_slower_keep_their_kernel(wins):
     assert [c for c, w in zip(SLOWER, wins(SLOWER)) if w] == []
 
