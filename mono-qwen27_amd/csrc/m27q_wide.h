@@ -60,7 +60,7 @@
 //     59 and 65;
 //   - the vector and matrix instructions of a wave pair add up (they hardly
 //     overlap): down's 543 vector instructions of 4 cycles and 64 MFMAs of 16 per
-//     unit (and set, of one per wave) are about 47 of its 65 us.  Dealing MFMAs
+//     unit (and set, of one per wave) are about 45 of its 65 us.  Dealing MFMAs
 //     between vector instructions of other groups (schedule groups, software
 //     pipelining over sets) was slower: 75 against 67 us on gate/up (traced);
 //   - loads must touch few 128-byte lines: a step of 4 groups reads each

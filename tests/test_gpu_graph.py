@@ -123,3 +123,72 @@ def test_decode_step_graph_replays_match_eager(m27q, ora, dev):
             torch.cuda.synchronize()
             for j, (t, w) in enumerate(zip(outs, want[i][0])):
                 assert np.array_equal(bits(t), w), (rep, i, j)
+
+
+def test_prefill_products_graph_replays_and_side_stream(m27q, ora, dev):
+    """Products of 9 to 40 rows (the wide kernel on one wave per slice, two and
+    four row waves, several weights in one launch; the VALU kernel's 16 rows;
+    two MFMA launches) and the split exact-dequantization products: on another
+    stream and in replays of a graph, bit for bit as eagerly, with the inputs
+    rewritten between the replays."""
+    import torch
+    W = {}
+    for name, t, rc, k, layout, seed in (
+            ("few", m27q.Q4_K, 1000, 2048, m27q.TILED, 1), ("mid", m27q.Q6_K, 8200, 2048, m27q.GGUF, 2),
+            ("many", m27q.Q5_K, 25000, 2048, m27q.TILED, 3), ("b", m27q.Q4_K, 9000, 2048, m27q.TILED, 4),
+            ("two", m27q.Q8_0, 4100, 2048, m27q.TILED, 5), ("valu", m27q.Q8_0, 25000, 2048, m27q.GGUF, 6),
+            ("f16", m27q.F16, 48, 2048, m27q.GGUF, 7)):
+        wb = (ora.quantize(t, np.random.default_rng(seed).standard_normal((rc, k)).astype(np.float32)) if t == m27q.F16
+              else ora.synth_weights(t, rc, k, seed=seed))
+        W[name] = m27q.Weight.upload(wb.reshape(-1), t, k // m27q.BLOCK_ELEMS[t], rc, layout, dev)
+    X = {M: torch.empty((M, 2048), dtype=torch.float32, device=dev) for M in (9, 20, 40)}
+    act = {M: m27q.Act(M, 2048, dev) for M in X}
+    calls = [(40, ["few"]), (40, ["few", "b"]), (40, ["mid"]), (20, ["many"]), (20, ["two"]), (9, ["valu"]), (20, ["few"])]
+    Ys = [[torch.empty((M, W[n].rc), dtype=torch.float32, device=dev) for n in names] for M, names in calls]
+    y = [torch.empty(W[n].rc, dtype=torch.float32, device=dev) for n in ("f16", "few")]
+    outs = [t for ys in Ys for t in ys] + y
+
+    def step(s):
+        for M in X:
+            m27q.quant_act(X[M], act[M], stream=s)
+        for (M, names), ys in zip(calls, Ys):
+            if len(names) == 1:
+                m27q.matmul_q8(W[names[0]], act[M], ys[0], stream=s)
+            else:
+                m27q.matmul_q8_multi([W[n] for n in names], act[M], ys, stream=s)
+        m27q.matvec_f32(W["f16"], X[9][0], y[0], stream=s)
+        m27q.matvec_f32(W["few"], X[9][1], y[1], stream=s)
+
+    def set_inputs(i):
+        for M in X:
+            X[M].copy_(torch.from_numpy(np.random.default_rng(100 * i + M).standard_normal((M, 2048)).astype(np.float32)))
+        for t in outs:
+            t.zero_()
+        torch.cuda.synchronize()
+
+    want = []
+    for i in range(3):
+        set_inputs(i)
+        say("prefill eager", i)
+        step(torch.cuda.current_stream())
+        want.append([bits(t) for t in outs])
+    side = torch.cuda.Stream()
+    set_inputs(1)
+    say("prefill side stream")
+    with torch.cuda.stream(side):
+        step(None)  # the current stream
+    side.synchronize()
+    for j, (t, w) in enumerate(zip(outs, want[1])):
+        assert np.array_equal(bits(t), w), j
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        step(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    for rep in range(2):
+        for i in (2, 0, 1):
+            set_inputs(i)
+            say("prefill replay", rep, i)
+            g.replay()
+            torch.cuda.synchronize()
+            for j, (t, w) in enumerate(zip(outs, want[i])):
+                assert np.array_equal(bits(t), w), (rep, i, j)
