@@ -46,8 +46,8 @@
 // What holds it back now, by the compiler's output (VGPRs, spills, instructions
 // and waits of the loops):
 //   - a step is conditional (slices differ by a unit), so the wait counts merge
-//     over both paths and each step drains every load in flight (vmcnt(0)) before
-//     its last groups: the weights are not a whole unit ahead in effect.  The next
+//     over both paths and every step waits once for all loads in flight
+//     (vmcnt(0)): the weights are not a whole unit ahead in effect.  The next
 //     unit's scales, needed by its first group, are asked for last;
 //   - Q6_K with four token tiles and three sets per wave (M = 49 to 64 past two
 //     sets per CU) does not fit 256 registers and spills 14 to 51 of them: 17408 x
